@@ -87,12 +87,36 @@ int wan_cross_attn(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out,
                    float softmax_scale, const int32_t* seqlen_k_dev, void* stream);
 
 /*
+ * The attention calls with optional scratch.  Where the query blocks leave the last round
+ * of workgroups mostly empty, their keys are split over the idle compute units, and the
+ * parts' fp32 results (O, running max, row sum) are merged by a second kernel; they go to
+ * `workspace`, 256-byte aligned, of wan_flash_attn_workspace() bytes (0: this size does not
+ * split).  With NULL or fewer bytes the call runs unsplit, as the entry point without _ws.
+ */
+size_t wan_flash_attn_workspace(int batch, int heads, int seqlen_q, int seqlen_k);
+int wan_flash_self_attn_ws(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out,
+                           int batch, int heads, int seqlen_q, int seqlen_k, int head_dim,
+                           float softmax_scale, int actual_seqlen_k,
+                           void* workspace, size_t workspace_bytes, void* stream);
+int wan_cross_attn_ws(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out,
+                      int batch, int heads, int seqlen_q, int seqlen_k, int head_dim,
+                      float softmax_scale, const int32_t* seqlen_k_dev,
+                      void* workspace, size_t workspace_bytes, void* stream);
+int wan_flash_attn_qnorm_ws(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out, int batch,
+                            int heads, int seqlen_q, int seqlen_k, int head_dim,
+                            const float* inv_rms_q, const void* gamma_q, const float* rope_cos,
+                            const float* rope_sin, float softmax_scale, const int32_t* seqlen_k_dev,
+                            void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Fused self-attention span of _FastBlock.forward, models/fast_dit.py:281-292:
  *   q,k = _tp_rms_qk(q, k) (RMS over all heads*128 channels of a token, eps,
  *         bf16 gamma [heads*128]); q,k = _rope(q), _rope(k); out = attention(q, k, v).
  * q, k, v are the raw projections [B, L, H, 128].  The per-token RMS of q and
- * the normalised, rotated k are written to `workspace` (at least
- * wan_self_attn_fused_workspace() bytes, 256-byte aligned); q is normalised
+ * the normalised, rotated k are written to `workspace` (256-byte aligned, of
+ * wan_self_attn_fused_workspace() bytes: an fp32 per token of q and a bf16 row per
+ * token of k, each rounded up to 256 bytes, which are needed, and after them the
+ * attention's split scratch, without which it runs unsplit); q is normalised
  * and rotated inside the attention kernel as it is loaded.
  */
 size_t wan_self_attn_fused_workspace(int batch, int heads, int seqlen);

@@ -39,6 +39,10 @@ SIGNATURES = {
     "wan_attn_init": (_I, []),
     "wan_flash_self_attn": (_I, [_T, _T, _T, _T, _I, _I, _I, _I, _I, _F, _I, _P]),
     "wan_cross_attn": (_I, [_T, _T, _T, _T, _I, _I, _I, _I, _I, _F, _P, _P]),
+    "wan_flash_attn_workspace": (_SZ, [_I, _I, _I, _I]),
+    "wan_flash_self_attn_ws": (_I, [_T, _T, _T, _T, _I, _I, _I, _I, _I, _F, _I, _P, _SZ, _P]),
+    "wan_cross_attn_ws": (_I, [_T, _T, _T, _T, _I, _I, _I, _I, _I, _F, _P, _P, _SZ, _P]),
+    "wan_flash_attn_qnorm_ws": (_I, [_T, _T, _T, _T, _I, _I, _I, _I, _I, _P, _P, _P, _P, _F, _P, _P, _SZ, _P]),
     "wan_self_attn_fused_workspace": (_SZ, [_I, _I, _I]),
     "wan_self_attn_fused": (_I, [_T, _T, _T, _T, _I, _I, _I, _I, _P, _P, _F, _P, _P, _F, _P, _SZ, _P]),
     "wan_cross_attn_fused_workspace": (_SZ, [_I, _I, _I]),

@@ -62,6 +62,24 @@ int check_scale(const char* fn, float scale) {
   return WAN_OK;
 }
 
+// The part of wan_self_attn_fused_workspace() that the call cannot do without: the inverse
+// RMS of q and the normalised, rotated k.
+size_t self_fused_bytes(int batch, int heads, int seqlen) {
+  if (batch <= 0 || heads <= 0 || seqlen <= 0) return 0;
+  const size_t rows = (size_t)batch * seqlen;
+  return align_up(rows * sizeof(float)) + align_up(rows * heads * kHeadDim * sizeof(bf16));
+}
+
+// Optional scratch of the attention's key split: used when given, aligned and large enough.
+int set_scratch(const char* fn, FlashArgs* a, void* scratch, size_t bytes) {
+  if (scratch == nullptr) return WAN_OK;
+  if (reinterpret_cast<uintptr_t>(scratch) % kAlign)
+    return set_error(WAN_ERR_INVALID, "%s: workspace must be 256-byte aligned", fn);
+  a->part = static_cast<float*>(scratch);
+  a->part_bytes = bytes;
+  return WAN_OK;
+}
+
 // Validates the arguments of one RMSNorm / statistics task and fills its PrepArgs.
 int rms_prep_args(const char* fn, wan_tensor x, void* out, int batch, int seqlen, int heads,
                   int head_dim, const void* gamma, float eps, const float* rope_cos,
@@ -110,9 +128,9 @@ const char* wan_attn_last_error(void) { return g_last_error; }
 
 int wan_attn_abi_version(void) { return 1; }
 
-int wan_flash_self_attn(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out, int batch,
-                        int heads, int seqlen_q, int seqlen_k, int head_dim, float softmax_scale,
-                        int actual_seqlen_k, void* stream) {
+int wan_flash_self_attn_ws(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out, int batch,
+                           int heads, int seqlen_q, int seqlen_k, int head_dim, float softmax_scale,
+                           int actual_seqlen_k, void* workspace, size_t workspace_bytes, void* stream) {
   const char* fn = "wan_flash_self_attn";
   int rc;
   if ((rc = check_scale(fn, softmax_scale))) return rc;
@@ -143,12 +161,20 @@ int wan_flash_self_attn(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out
   a.seqlen_all = actual_seqlen_k;
   a.scale = softmax_scale;
   a.qprep = kQPlain;
+  if ((rc = set_scratch(fn, &a, workspace, workspace_bytes))) return rc;
   return launch_flash_fwd(a, static_cast<hipStream_t>(stream));
 }
 
-int wan_cross_attn(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out, int batch, int heads,
-                   int seqlen_q, int seqlen_k, int head_dim, float softmax_scale,
-                   const int32_t* seqlen_k_dev, void* stream) {
+int wan_flash_self_attn(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out, int batch,
+                        int heads, int seqlen_q, int seqlen_k, int head_dim, float softmax_scale,
+                        int actual_seqlen_k, void* stream) {
+  return wan_flash_self_attn_ws(q, k, v, out, batch, heads, seqlen_q, seqlen_k, head_dim,
+                                softmax_scale, actual_seqlen_k, nullptr, 0, stream);
+}
+
+int wan_cross_attn_ws(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out, int batch, int heads,
+                      int seqlen_q, int seqlen_k, int head_dim, float softmax_scale,
+                      const int32_t* seqlen_k_dev, void* workspace, size_t workspace_bytes, void* stream) {
   const char* fn = "wan_cross_attn";
   int rc;
   if ((rc = check_scale(fn, softmax_scale))) return rc;
@@ -173,13 +199,23 @@ int wan_cross_attn(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out, int
   a.seqlen_all = seqlen_k;
   a.scale = softmax_scale;
   a.qprep = kQPlain;
+  if ((rc = set_scratch(fn, &a, workspace, workspace_bytes))) return rc;
   return launch_flash_fwd(a, static_cast<hipStream_t>(stream));
 }
 
+int wan_cross_attn(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out, int batch, int heads,
+                   int seqlen_q, int seqlen_k, int head_dim, float softmax_scale,
+                   const int32_t* seqlen_k_dev, void* stream) {
+  return wan_cross_attn_ws(q, k, v, out, batch, heads, seqlen_q, seqlen_k, head_dim, softmax_scale,
+                           seqlen_k_dev, nullptr, 0, stream);
+}
+
+size_t wan_flash_attn_workspace(int batch, int heads, int seqlen_q, int seqlen_k) {
+  return flash_split_bytes(batch, heads, seqlen_q, seqlen_k);
+}
+
 size_t wan_self_attn_fused_workspace(int batch, int heads, int seqlen) {
-  if (batch <= 0 || heads <= 0 || seqlen <= 0) return 0;
-  const size_t rows = (size_t)batch * seqlen;
-  return align_up(rows * sizeof(float)) + align_up(rows * heads * kHeadDim * sizeof(bf16));
+  return self_fused_bytes(batch, heads, seqlen) + flash_split_bytes(batch, heads, seqlen, seqlen);
 }
 
 int wan_rms_norm(wan_tensor x, void* out, int batch, int seqlen, int heads, int head_dim,
@@ -239,11 +275,11 @@ int wan_rms_norm_qk_sumsq(wan_tensor k, void* k_out, int batch, int seqlen, int 
   return launch_rms_prep2(aq, ak, static_cast<hipStream_t>(stream));
 }
 
-int wan_flash_attn_qnorm(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out, int batch,
-                         int heads, int seqlen_q, int seqlen_k, int head_dim,
-                         const float* inv_rms_q, const void* gamma_q, const float* rope_cos,
-                         const float* rope_sin, float softmax_scale, const int32_t* seqlen_k_dev,
-                         void* stream) {
+int wan_flash_attn_qnorm_ws(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out, int batch,
+                            int heads, int seqlen_q, int seqlen_k, int head_dim,
+                            const float* inv_rms_q, const void* gamma_q, const float* rope_cos,
+                            const float* rope_sin, float softmax_scale, const int32_t* seqlen_k_dev,
+                            void* workspace, size_t workspace_bytes, void* stream) {
   const char* fn = "wan_flash_attn_qnorm";
   int rc;
   if ((rc = check_scale(fn, softmax_scale))) return rc;
@@ -279,7 +315,18 @@ int wan_flash_attn_qnorm(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor ou
   a.gamma_q = static_cast<const bf16*>(gamma_q);
   a.cos = rope_cos;
   a.sin = rope_sin;
+  if ((rc = set_scratch(fn, &a, workspace, workspace_bytes))) return rc;
   return launch_flash_fwd(a, static_cast<hipStream_t>(stream));
+}
+
+int wan_flash_attn_qnorm(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out, int batch,
+                         int heads, int seqlen_q, int seqlen_k, int head_dim,
+                         const float* inv_rms_q, const void* gamma_q, const float* rope_cos,
+                         const float* rope_sin, float softmax_scale, const int32_t* seqlen_k_dev,
+                         void* stream) {
+  return wan_flash_attn_qnorm_ws(q, k, v, out, batch, heads, seqlen_q, seqlen_k, head_dim, inv_rms_q,
+                                 gamma_q, rope_cos, rope_sin, softmax_scale, seqlen_k_dev, nullptr, 0,
+                                 stream);
 }
 
 int wan_self_attn_fused(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out, int batch,
@@ -301,7 +348,7 @@ int wan_self_attn_fused(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out
   if (!aligned16(gamma_q) || !aligned16(gamma_k) || !aligned16(rope_cos) || !aligned16(rope_sin))
     return set_error(WAN_ERR_INVALID, "%s: gamma and rope tables must be 16-byte aligned", fn);
   if (!(eps >= 0.f)) return set_error(WAN_ERR_INVALID, "%s: eps must be >= 0", fn);
-  const size_t need = wan_self_attn_fused_workspace(batch, heads, seqlen);
+  const size_t need = self_fused_bytes(batch, heads, seqlen);
   if (workspace == nullptr || workspace_bytes < need)
     return set_error(WAN_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", fn, need,
                      workspace ? workspace_bytes : (size_t)0);
@@ -314,8 +361,9 @@ int wan_self_attn_fused(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out
   if ((rc = wan_rms_norm_qk(q, k, khat, batch, seqlen, heads, head_dim, gamma_k, eps, rope_cos,
                             rope_sin, inv_q, stream)))
     return rc;
-  return wan_flash_attn_qnorm(q, kt, v, out, batch, heads, seqlen, seqlen, head_dim, inv_q, gamma_q,
-                              rope_cos, rope_sin, softmax_scale, nullptr, stream);
+  return wan_flash_attn_qnorm_ws(q, kt, v, out, batch, heads, seqlen, seqlen, head_dim, inv_q, gamma_q,
+                                 rope_cos, rope_sin, softmax_scale, nullptr,
+                                 static_cast<char*>(workspace) + need, workspace_bytes - need, stream);
 }
 
 size_t wan_cross_attn_fused_workspace(int batch, int heads, int seqlen_q) {

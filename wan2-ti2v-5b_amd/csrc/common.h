@@ -70,8 +70,17 @@ struct FlashArgs {
   const bf16* gamma_q;      // [H*128]
   const float* cos;         // [Lq, 64] (kQNormRope)
   const float* sin;
+  // Key-split of the last, partly filled round of workgroups: blocks before split_from are
+  // whole, each block from there on is `splits` workgroups over a part of its keys that
+  // leave their fp32 O, m and l in `part` (null: no split).  Set by the launcher from
+  // `part` and `part_bytes`, the scratch the caller gave.
+  float* part;
+  size_t part_bytes;
+  int split_from, splits;
 };
 int launch_flash_fwd(const FlashArgs& a, hipStream_t s);
+// Scratch bytes that a launch of this size makes use of (0: it does not split).
+size_t flash_split_bytes(int B, int H, int Lq, int Lk);
 // CU count of the current device (cached per device after the first query).
 int device_cu_count();
 

@@ -459,7 +459,34 @@ struct TileCore {
   }
 };
 
-template <int NW, int QP>
+// Which (batch, head) and query block a block number stands for.  One key length for all:
+// (b, h) major, the query blocks of one head run together on one XCD and share its K/V
+// through that XCD's L2.  Per-sample key lengths: batch fastest, so every XCD receives the
+// same mix of long and short samples (the K/V of these calls are small).
+struct BlockId {
+  int mblk, b, h;
+};
+__device__ __forceinline__ BlockId block_id(const FlashArgs& a, int pid, int num_m) {
+  BlockId r;
+  if (a.seqlen_k == nullptr) {
+    r.mblk = pid % num_m;
+    const int bh = pid / num_m;
+    r.b = bh / a.H;
+    r.h = bh - r.b * a.H;
+  } else {
+    r.b = pid % a.B;
+    const int rest = pid / a.B;
+    r.mblk = rest % num_m;
+    r.h = rest / num_m;
+  }
+  return r;
+}
+
+// A split part's result: per wave (32 query rows) 16 groups of 64 x 4 fp32 (group 4 md + g
+// holds o[md][4g..4g+3] of every lane, so that one store writes 1 KB), then m and l per lane.
+constexpr int kPartFloats = 64 * 64 + 128;
+
+template <int NW, int QP, bool SPLIT>
 __global__ __launch_bounds__(NW * 64, 2) void flash_fwd_kernel(const FlashArgs a) {
   constexpr int BM = NW * 32;
 
@@ -480,26 +507,25 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_fwd_kernel(const FlashArgs a
   const int n32 = lane & 31, hh = lane >> 5;
 
   const int num_m = (a.Lq + BM - 1) / BM;
-  const int pid = xcd_remap(blockIdx.x, gridDim.x);
-  int mblk, b, h;
-  if (a.seqlen_k == nullptr) {
-    // (b, h) major: the query blocks of one head run together on one XCD and
-    // share its K/V through that XCD's L2
-    mblk = pid % num_m;
-    const int bh = pid / num_m;
-    b = bh / a.H;
-    h = bh - b * a.H;
+  int pid, part = -1;   // part: this workgroup's number among the split parts
+  if (!SPLIT || (int)blockIdx.x < a.split_from) {
+    pid = xcd_remap(blockIdx.x, SPLIT ? a.split_from : gridDim.x);
   } else {
-    // per-sample key lengths: batch fastest, so every XCD receives the same
-    // mix of long and short samples (the K/V of these calls are small)
-    b = pid % a.B;
-    const int rest = pid / a.B;
-    mblk = rest % num_m;
-    h = rest / num_m;
+    part = xcd_remap(blockIdx.x - a.split_from, gridDim.x - a.split_from);
+    pid = a.split_from + part / a.splits;
   }
+  const BlockId blk = block_id(a, pid, num_m);
+  const int mblk = blk.mblk, b = blk.b, h = blk.h;
 
   int len = a.seqlen_all;
   if (a.seqlen_k != nullptr) len = min(max(a.seqlen_k[b], 0), a.Lk);
+  // the keys of this workgroup: all, or part `part % splits` of the tiles
+  int64_t key0 = 0;
+  if (SPLIT && part >= 0) {
+    const int nt = (len + BN - 1) / BN, i = part % a.splits;
+    key0 = (nt * i / a.splits) * BN;
+    len = min(len, (nt * (i + 1) / a.splits) * BN) - (int)key0;
+  }
   const int ntiles = (len + BN - 1) / BN;
 
   const int qrow = mblk * BM + wave * 32 + n32;
@@ -508,8 +534,8 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_fwd_kernel(const FlashArgs a
 
   if (ntiles > 0) {
     TileLoader<NW> kl, vl;
-    kl.init(a.k.ptr + b * a.k.sb + h * a.k.sh, a.k.st, wave, lane, true);
-    vl.init(a.v.ptr + b * a.v.sb + h * a.v.sh, a.v.st, wave, lane, false);
+    kl.init(a.k.ptr + b * a.k.sb + h * a.k.sh + (SPLIT ? key0 * a.k.st : 0), a.k.st, wave, lane, true);
+    vl.init(a.v.ptr + b * a.v.sb + h * a.v.sh + (SPLIT ? key0 * a.v.st : 0), a.v.st, wave, lane, false);
     // RoPE tables: this wave's 32 cos and sin rows go through LDS and are read
     // back per lane.  With the ring of four they use buffers 1-3 and the extra
     // 32 KB while K0 and V0 are already being copied; with two buffers they use
@@ -671,6 +697,21 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_fwd_kernel(const FlashArgs a
     if constexpr (RING == 4) __syncthreads();
   }
 
+  if (SPLIT && part >= 0) {
+    if (mblk * BM + wave * 32 >= a.Lq) return;
+    float* p = a.part + ((int64_t)part * NW + wave) * kPartFloats;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = c.o[i >> 2][4 * (i & 3) + e];
+      *reinterpret_cast<f32x4*>(p + i * 256 + lane * 4) = v;
+    }
+    p[4096 + lane] = c.m_run;
+    p[4160 + lane] = c.l_run;
+    return;
+  }
+
   // Output store, staged through the K buffers: they are free here (their last
   // reads came before the last barrier, and no load into them is in flight).
   bf16* stage = (wave < 4 ? k_lds[0] : k_lds[1]) + (wave & 3) * 2048;
@@ -679,12 +720,61 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_fwd_kernel(const FlashArgs a
 
 // Explicit instantiations: without them clang emits the host launch stubs of
 // only some of these (lambda-using) kernel template instances.
-template __global__ void flash_fwd_kernel<kWaves, kQPlain>(const FlashArgs);
-template __global__ void flash_fwd_kernel<kWaves, kQNorm>(const FlashArgs);
-template __global__ void flash_fwd_kernel<kWaves, kQNormRope>(const FlashArgs);
-template __global__ void flash_fwd_kernel<4, kQPlain>(const FlashArgs);
-template __global__ void flash_fwd_kernel<4, kQNorm>(const FlashArgs);
-template __global__ void flash_fwd_kernel<4, kQNormRope>(const FlashArgs);
+template __global__ void flash_fwd_kernel<kWaves, kQPlain, false>(const FlashArgs);
+template __global__ void flash_fwd_kernel<kWaves, kQNorm, false>(const FlashArgs);
+template __global__ void flash_fwd_kernel<kWaves, kQNormRope, false>(const FlashArgs);
+template __global__ void flash_fwd_kernel<kWaves, kQPlain, true>(const FlashArgs);
+template __global__ void flash_fwd_kernel<kWaves, kQNorm, true>(const FlashArgs);
+template __global__ void flash_fwd_kernel<kWaves, kQNormRope, true>(const FlashArgs);
+template __global__ void flash_fwd_kernel<4, kQPlain, false>(const FlashArgs);
+template __global__ void flash_fwd_kernel<4, kQNorm, false>(const FlashArgs);
+template __global__ void flash_fwd_kernel<4, kQNormRope, false>(const FlashArgs);
+
+// The output rows of the split blocks: O = sum_i w_i O_i / sum_i w_i l_i with
+// w_i = exp2(m_i - max m).  One workgroup per 32 rows, one wave per 32 channels; a part
+// without keys (l = 0, m = -inf) weighs nothing, and rows without any key are zeros.
+__global__ __launch_bounds__(256) void flash_merge_kernel(const FlashArgs a) {
+  constexpr int NW = kWaves, BM = NW * 32;
+  __shared__ __attribute__((aligned(16))) bf16 rows[32 * D];
+  const int lane = threadIdx.x & 63, md = threadIdx.x >> 6;
+  const int n32 = lane & 31, hh = lane >> 5;
+  const int blk = blockIdx.x / NW, wave = blockIdx.x % NW;
+  const BlockId id = block_id(a, a.split_from + blk, (a.Lq + BM - 1) / BM);
+  const int row0 = id.mblk * BM + wave * 32;
+  if (row0 >= a.Lq) return;
+
+  const float* p0 = a.part + ((int64_t)blk * a.splits * NW + wave) * kPartFloats;
+  const int64_t next = (int64_t)NW * kPartFloats;
+  float m = -INFINITY;
+  for (int i = 0; i < a.splits; ++i) m = fmaxf(m, p0[i * next + 4096 + lane]);
+  f32x4 o[4] = {};
+  float l = 0.f;
+  for (int i = 0; i < a.splits; ++i) {
+    const float* p = p0 + i * next;
+    const float li = p[4160 + lane], mi = p[4096 + lane];
+    const float w = li == 0.f && mi == -INFINITY ? 0.f : fast_exp2(mi - m);
+    l += w * li;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) o[g] += w * *reinterpret_cast<const f32x4*>(p + (4 * md + g) * 256 + lane * 4);
+  }
+  const float l_tot = pair_sum(l);
+  const float inv_l = l_tot > 0.f ? 1.f / l_tot : 0.f;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    bf16x4 w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = (bf16)(o[g][e] * inv_l);
+    *reinterpret_cast<bf16x4*>(rows + n32 * D + 32 * md + 8 * g + 4 * hh) = w;
+  }
+  __syncthreads();
+  bf16* out = a.o + id.b * a.o_sb + id.h * a.o_sh;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int r = (threadIdx.x >> 4) + 16 * j, c = (threadIdx.x & 15) * 8;
+    if (row0 + r < a.Lq)
+      *reinterpret_cast<bf16x8*>(out + (int64_t)(row0 + r) * a.o_st + c) = *reinterpret_cast<const bf16x8*>(rows + r * D + c);
+  }
+}
 
 // ---------------------------------------------------------------------------
 // Short keys (<= kShortKeys, the cross-attention's text keys) with per-sample key
@@ -921,22 +1011,70 @@ int launch_short(const FlashArgs& a, hipStream_t s) {
   return e == hipSuccess ? 0 : set_error(4, "flash_fwd launch: %s", hipGetErrorString(e));
 }
 
+// Up to this many keys (the cross-attention's 512 text keys) a workgroup has 4
+// waves (128 rows) and two run per CU: with only a few tiles per workgroup, one
+// workgroup's start-up (Q load, first tile loads) then overlaps the other's
+// tiles (measured 5% faster at 512 keys; equal or slower from 1080 keys on).
+constexpr int kShortKeys = 1024;
+
+// How the 8-wave kernel's last round of workgroups (one per CU) is split.  When the blocks
+// leave `rem` of them for a last round and that fills half of the CUs at most, each of
+// those is run as n workgroups over a part of the keys and merged.  A tile less costs ~1.4 us
+// less; a split costs ~5 us (the merge launch, the parts' own start) and 0.05 us per part
+// (132 KB of fp32 written and read).  Self-attention, batch 2, 24 heads, us unsplit / split:
+//   1500 tokens (rem 32, n 8)  107.6 / 92.6      2048 (rem 128, n 2)  139.4 / 132.8
+//   4114 (rem 48, n 5)         482.1 / 437.3
+// More than one round of parts loses: 4862 tokens (rem 144) 576 / 581 at n 3, 7854 (rem 208)
+// 1382 / 1411 at n 2 -- while a last round is partly idle the busy CUs clock higher.
+struct SplitPlan {
+  int from, blocks, splits;   // whole blocks, split blocks, parts of each
+  size_t bytes;
+};
+constexpr int kMaxSplits = 8;
+SplitPlan split_plan(int B, int H, int Lq, int Lk) {
+  SplitPlan p{0, 0, 1, 0};
+  const int64_t blocks = (int64_t)((Lq + kWaves * 32 - 1) / (kWaves * 32)) * B * H;
+  const int cus = device_cu_count();
+  const int rem = (int)(blocks % cus), nt = (Lk + BN - 1) / BN;
+  if (rem == 0 || blocks > 0x7fffffff) return p;
+  float best = 0.f;
+  for (int n = 2; n <= kMaxSplits && rem * n <= cus && n <= nt; ++n) {
+    const float gain = 1.4f * (nt - (nt + n - 1) / n) - 5.f - 0.05f * (rem * n);
+    if (gain > best) {
+      best = gain;
+      p.splits = n;
+    }
+  }
+  if (p.splits < 2) return p;
+  p.from = (int)(blocks - rem);
+  p.blocks = rem;
+  p.bytes = (size_t)rem * p.splits * kWaves * kPartFloats * sizeof(float);
+  return p;
+}
+
 template <int NW, int QP>
 int launch_nw(const FlashArgs& a, hipStream_t s) {
   constexpr int BM = NW * 32;
   const int64_t num_m = (a.Lq + BM - 1) / BM;
   const int64_t grid = num_m * a.B * a.H;
   if (grid > 0x7fffffff) return set_error(2, "flash_fwd: grid of %lld workgroups too large", (long long)grid);
-  hipLaunchKernelGGL((flash_fwd_kernel<NW, QP>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
+  if constexpr (NW == kWaves) {
+    const SplitPlan p = split_plan(a.B, a.H, a.Lq, a.seqlen_k != nullptr ? a.Lk : a.seqlen_all);
+    if (p.splits > 1 && a.part != nullptr && a.part_bytes >= p.bytes) {
+      FlashArgs as = a;
+      as.split_from = p.from;
+      as.splits = p.splits;
+      hipLaunchKernelGGL((flash_fwd_kernel<NW, QP, true>), dim3((unsigned)(p.from + p.blocks * p.splits)),
+                         dim3(NW * 64), 0, s, as);
+      hipLaunchKernelGGL(flash_merge_kernel, dim3((unsigned)p.blocks * NW), dim3(256), 0, s, as);
+      const hipError_t e = hipGetLastError();
+      return e == hipSuccess ? 0 : set_error(4, "flash_fwd launch: %s", hipGetErrorString(e));
+    }
+  }
+  hipLaunchKernelGGL((flash_fwd_kernel<NW, QP, false>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : set_error(4, "flash_fwd launch: %s", hipGetErrorString(e));
 }
-
-// Up to this many keys (the cross-attention's 512 text keys) a workgroup has 4
-// waves (128 rows) and two run per CU: with only a few tiles per workgroup, one
-// workgroup's start-up (Q load, first tile loads) then overlaps the other's
-// tiles (measured 5% faster at 512 keys; equal or slower from 1080 keys on).
-constexpr int kShortKeys = 1024;
 
 // With per-sample key lengths the items of a short-key call differ in cost, and
 // those of the short samples are mostly start-up: there the persistent kernel,
@@ -972,6 +1110,11 @@ int device_cu_count() {
     cus[dev] = n;
   }
   return cus[dev];
+}
+
+size_t flash_split_bytes(int B, int H, int Lq, int Lk) {
+  if (B <= 0 || H <= 0 || Lq <= 0 || Lk <= kShortKeys) return 0;
+  return split_plan(B, H, Lq, Lk).bytes;
 }
 
 int launch_flash_fwd(const FlashArgs& a, hipStream_t s) {

@@ -74,6 +74,17 @@ def _seqlen_ptr(fn: str, seqlen_k: Optional[torch.Tensor], B: int, device) -> in
     return seqlen_k.data_ptr()
 
 
+def _split_scratch(lib, q: torch.Tensor, Lk: int):
+    """Scratch of the attention's key split for q [B, Lq, H, 128] against Lk keys: (tensor to
+    keep until the launch, address, bytes); without one at sizes that do not split."""
+    B, Lq, H, _ = q.shape
+    n = lib.wan_flash_attn_workspace(B, H, Lq, Lk)
+    if n == 0:
+        return None, None, 0
+    t = torch.empty(n, dtype=torch.uint8, device=q.device)
+    return t, t.data_ptr(), n
+
+
 # ---------------------------------------------------------------------------
 # self-attention (kernels/self_attention_nst.py:49-117; models/fast_dit.py:186-207)
 # ---------------------------------------------------------------------------
@@ -88,10 +99,12 @@ def flash_self_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if actual_seqlen_k > Lk:
         raise ValueError(f"{fn}: actual_seqlen_k must be in (0, {Lk}], got {actual_seqlen_k}")
     out = torch.empty((B, Lq, H, D), dtype=q.dtype, device=q.device)
+    lib = N.lib()
     with torch.cuda.device(q.device):
-        N.check("wan_flash_self_attn", N.lib().wan_flash_self_attn(
+        ws, ws_ptr, ws_bytes = _split_scratch(lib, q, Lk)
+        N.check("wan_flash_self_attn", lib.wan_flash_self_attn_ws(
             N.tensor4(q), N.tensor4(k), N.tensor4(v), N.tensor4(out), B, H, Lq, Lk, D,
-            float(softmax_scale), int(actual_seqlen_k), _stream(q.device)))
+            float(softmax_scale), int(actual_seqlen_k), ws_ptr, ws_bytes, _stream(q.device)))
     return out
 
 
@@ -109,10 +122,12 @@ def cross_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     Lk = k.shape[1]
     sk = _seqlen_ptr(fn, seqlen_k, B, q.device)
     out = torch.empty((B, Lq, H, D), dtype=q.dtype, device=q.device)
+    lib = N.lib()
     with torch.cuda.device(q.device):
-        N.check("wan_cross_attn", N.lib().wan_cross_attn(
+        ws, ws_ptr, ws_bytes = _split_scratch(lib, q, Lk)
+        N.check("wan_cross_attn", lib.wan_cross_attn_ws(
             N.tensor4(q), N.tensor4(k), N.tensor4(v), N.tensor4(out), B, H, Lq, Lk, D,
-            float(softmax_scale), sk, _stream(q.device)))
+            float(softmax_scale), sk, ws_ptr, ws_bytes, _stream(q.device)))
     return out
 
 
@@ -138,10 +153,10 @@ def self_attn_fused(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     _check_vec(fn, "gamma_k", gamma_k, H * D, torch.bfloat16, q.device)
     _check_rope(fn, cos, sin, L, q.device)
     lib = N.lib()
-    ws = torch.empty(max(1, lib.wan_self_attn_fused_workspace(B, H, L)), dtype=torch.uint8,
-                     device=q.device)
     out = torch.empty((B, L, H, D), dtype=q.dtype, device=q.device)
     with torch.cuda.device(q.device):
+        ws = torch.empty(max(1, lib.wan_self_attn_fused_workspace(B, H, L)), dtype=torch.uint8,
+                         device=q.device)
         N.check("wan_self_attn_fused", lib.wan_self_attn_fused(
             N.tensor4(q), N.tensor4(k), N.tensor4(v), N.tensor4(out), B, H, L, D,
             gamma_q.data_ptr(), gamma_k.data_ptr(), float(eps), cos.data_ptr(), sin.data_ptr(),
@@ -267,12 +282,14 @@ def flash_attn_qnorm(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, inv_rms_
         _check_rope(fn, cos, sin, Lq, q.device)
     sk = _seqlen_ptr(fn, seqlen_k, B, q.device)
     out = torch.empty((B, Lq, H, D), dtype=q.dtype, device=q.device)
+    lib = N.lib()
     with torch.cuda.device(q.device):
-        N.check("wan_flash_attn_qnorm", N.lib().wan_flash_attn_qnorm(
+        ws, ws_ptr, ws_bytes = _split_scratch(lib, q, Lk)
+        N.check("wan_flash_attn_qnorm", lib.wan_flash_attn_qnorm_ws(
             N.tensor4(q), N.tensor4(k), N.tensor4(v), N.tensor4(out), B, H, Lq, Lk, D,
             inv_rms_q.data_ptr(), gamma_q.data_ptr(),
             None if cos is None else cos.data_ptr(), None if sin is None else sin.data_ptr(),
-            float(softmax_scale), sk, _stream(q.device)))
+            float(softmax_scale), sk, ws_ptr, ws_bytes, _stream(q.device)))
     return out
 
 
@@ -413,13 +430,14 @@ def self_attn_fused_sumsq(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sum
     out = torch.empty((B, L, H, D), dtype=q.dtype, device=q.device)
     s = _stream(q.device)
     with torch.cuda.device(q.device):
+        ws, ws_ptr, ws_bytes = _split_scratch(lib, q, L)
         N.check("wan_rms_norm_qk_sumsq", lib.wan_rms_norm_qk_sumsq(
             N.tensor4(k), khat.data_ptr(), B, L, H, D, gamma_k.data_ptr(), float(eps),
             cos.data_ptr(), sin.data_ptr(), sumsq.data_ptr(), inv.data_ptr(), s))
-        N.check("wan_flash_attn_qnorm", lib.wan_flash_attn_qnorm(
+        N.check("wan_flash_attn_qnorm", lib.wan_flash_attn_qnorm_ws(
             N.tensor4(q), N.tensor4(khat), N.tensor4(v), N.tensor4(out), B, H, L, L, D,
             inv.data_ptr(), gamma_q.data_ptr(), cos.data_ptr(), sin.data_ptr(),
-            float(softmax_scale), None, s))
+            float(softmax_scale), None, ws_ptr, ws_bytes, s))
     return out
 
 
