@@ -8,23 +8,28 @@
 // models/fast_dit.py:134-147) are 48 + 48 partial sums read by the K pass, and q is
 // not read again before the attention kernel.
 //
-// Design: 256 x 256 output tile per workgroup, 8 waves in a 2 x 4 grid, each wave
-// 128 (m) x 64 (n): 8 accumulators of v_mfma_f32_32x32x16_bf16, two waves per SIMD.
-// The MFMA computes out^T tiles, w rows on the MFMA row axis and x rows on the column
-// axis, so a lane holds one output row (lane % 32) and half of each 64-column block: a
-// 64-column sum of squares is lane-local plus one exchange with the lane 32 apart, as
-// the attention kernel's softmax row sums are.  K advances 64 per tile; the 256 x 64
-// tiles of x and w (32 KB each) go global -> LDS by 16-byte copies into rows of eight
-// 16-byte chunks, chunk c of row r at position c ^ ((r / 2) % 8) (conflict-free operand
-// reads), in two slots, one barrier per tile.  Program order is pinned MFMA by MFMA:
-// each MFMA is followed by one fragment read of the next k-step and, in a tile's first
-// k-step, one copy of the next tile, and the barrier sits inside the last k-step so the
-// next tile's first reads overlap its remaining MFMAs.  Workgroups run in groups of 8
-// M-tiles per N-tile, each XCD owning a contiguous range, so the tiles running together
-// on an XCD share x and w rows in its L2.
+// Design: GBM x 256 output tile per workgroup (GBM 128, 192, 256 or 320: the launcher
+// takes the height that fills the rounds of workgroups best), 8 waves in a 2 x 4 grid,
+// each wave GBM/2 (m) x 64 (n): up to 10 accumulators of v_mfma_f32_32x32x16_bf16, two
+// waves per SIMD.  The MFMA computes out^T tiles, w rows on the MFMA row axis and x rows
+// on the column axis, so a lane holds one output row (lane % 32) and half of each
+// 64-column block: a 64-column sum of squares is lane-local plus one exchange with the
+// lane 32 apart, as the attention kernel's softmax row sums are.  K advances 64 per
+// tile; the GBM x 64 and 256 x 64 tiles of x and w (32 KB for 256 rows) go global -> LDS
+// by 16-byte copies into rows of eight 16-byte chunks, chunk c of row r at position c ^
+// ((r / 2) % 8) (conflict-free operand reads), in two slots (three with 128 rows, whose
+// 1024 MFMA cycles per tile are less than a copy takes: 46 -> 33 us at M 256), one
+// barrier per tile.  (256 rows in 32-k stages, three to five slots: 4-8% slower than 64
+// k in two.) Program order is pinned MFMA by MFMA: each MFMA is followed by one fragment
+// read of the next k-step and, in a tile's first k-step, one copy of a coming tile, and
+// the barrier sits inside the last k-step so the next tile's first reads overlap its
+// remaining MFMAs.  Workgroups run in groups of 8 M-tiles per N-tile, each XCD owning a
+// contiguous range, so the tiles running together on an XCD share x and w rows in its
+// L2.
 //
-// At the QKV shape (M 15708, N 9216, K 3072) it reaches 1.28-1.31 PFLOP/s, 86-88% of
-// hipBLASLt's F.linear timed beside it, with output bit-identical.  Both are power
+// At the QKV shape (M 15708, N 9216, K 3072; 256 rows) it reaches 1.28-1.31 PFLOP/s,
+// 86-88% of hipBLASLt's F.linear timed beside it, with output bit-identical; at M 2160
+// (320 rows) 1.29 PFLOP/s against hipBLASLt's 1.17.  Both are power
 // limited (all-zero operands run either ~25% faster); on zeros this kernel's k-loop is
 // ~13% slower per tile than hipBLASLt's.  4 waves of 128 x 128 (a third less LDS read
 // traffic, one wave per SIMD) run the loop at a higher clock (1.72 vs 1.58 GHz) but in
@@ -37,9 +42,9 @@ namespace wan {
 
 namespace {
 
-constexpr int GBM = 256, GBN = 256;
+constexpr int GBN = 256;
 constexpr int kGroupM = 8;
-// 8 waves in a 2 x 4 grid (each 128 x 64 of the 256 x 256 tile, two waves per SIMD),
+// 8 waves in a 2 x 4 grid (each 128 x 64 of a 256 x 256 tile, two waves per SIMD),
 // 64 k per stage: measured the fastest of 2 x 2 / 2 x 4 waves, 32 / 64 k, 2-5 stages
 constexpr int kGemmWM = 2, kGemmWN = 4, kGemmBK = 64;
 
@@ -68,7 +73,7 @@ __device__ __forceinline__ float pair_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-template <int WM, int WN, int BK>
+template <int WM, int WN, int BK, int GBM>
 struct GemmCfg {
   static constexpr int kWaves = WM * WN;
   static constexpr int kThreads = 64 * kWaves;
@@ -76,44 +81,42 @@ struct GemmCfg {
   static constexpr int TN = GBN / WN / 32;        // 32-row blocks of w (output columns) per wave
   static constexpr int kCpr = BK / 8;             // 16-byte chunks per tile row
   static constexpr int kRps = 16 / kCpr;          // rows per 256-byte bank sweep
-  static constexpr int kTileElems = 256 * BK;
-  static constexpr int kBlocks = kTileElems / 512; // 1 KB copies per tile
-  static constexpr int kPerWave = kBlocks / kWaves;
   static constexpr int kRowsPerBlock = 512 / BK;  // tile rows per 1 KB copy
-  static_assert(kBlocks % kWaves == 0, "copies must divide over the waves");
+  static constexpr int kXPerWave = GBM / kRowsPerBlock / kWaves;  // 1 KB copies per wave and tile
+  static constexpr int kWPerWave = GBN / kRowsPerBlock / kWaves;
+  static_assert(GBM % (32 * WM) == 0 && GBN % (64 * WN) == 0, "whole 32-row and 64-column blocks");
+  static_assert(GBM % (kRowsPerBlock * kWaves) == 0 && GBN % (kRowsPerBlock * kWaves) == 0,
+                "copies must divide over the waves");
+  static_assert(2 * GBM * BK >= kWaves * 32 * GBN / WN, "the x tiles hold the output staging");
   // chunk c of row r sits at position c ^ ((r / kRps) % kCpr): the 16 rows read by a
   // 16-lane phase of an operand read land on 16 distinct 16-byte bank groups
   __device__ static __forceinline__ int swz(int row) { return (row / kRps) & (kCpr - 1); }
 };
 
-// Copies of one 256 x BK tile in 1 KB blocks, wave w issuing blocks w, w + waves, ...
+// Copies of one tile of 8 N x BK rows in 1 KB blocks, N per wave, wave w issuing blocks w, w + waves, ...
 // Lane l fills LDS row (block rows) + l / kCpr, position l % kCpr, with the global chunk
 // the row's swizzle puts there.  Offsets are bytes from the tile's (row 0, k 0).
-template <class C>
+template <class C, int N>
 struct GemmTileLoader {
-  uint32_t off[C::kPerWave];
+  uint32_t off[N];
   __device__ void init(int64_t ld, int rows_valid, int wave, int lane) {
 #pragma unroll
-    for (int i = 0; i < C::kPerWave; ++i) {
+    for (int i = 0; i < N; ++i) {
       const int row = C::kRowsPerBlock * (wave + C::kWaves * i) + lane / C::kCpr;
       const int r = min(row, rows_valid - 1);       // rows past the matrix repeat its last row
       off[i] = (uint32_t)((int64_t)r * ld * 2 + (((lane % C::kCpr) ^ C::swz(row)) << 4));
     }
-  }
-  __device__ __forceinline__ void issue(const char* tile_base, bf16* dst, int wave) const {
-#pragma unroll
-    for (int i = 0; i < C::kPerWave; ++i) issue_one(tile_base, dst, wave, i);
   }
   __device__ __forceinline__ void issue_one(const char* tile_base, bf16* dst, int wave, int i) const {
     dma16(tile_base, off[i], lds_addr(dst + (wave + C::kWaves * i) * 512));
   }
 };
 
-template <int WM, int WN, int BK>
+template <int WM, int WN, int BK, int GBM, int SLOTS>
 __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmArgs a) {
-  using C = GemmCfg<WM, WN, BK>;
-  __shared__ __attribute__((aligned(1024))) bf16 xs[2][C::kTileElems];
-  __shared__ __attribute__((aligned(1024))) bf16 ws[2][C::kTileElems];
+  using C = GemmCfg<WM, WN, BK, GBM>;
+  __shared__ __attribute__((aligned(1024))) bf16 xs[SLOTS][GBM * BK];
+  __shared__ __attribute__((aligned(1024))) bf16 ws[SLOTS][GBN * BK];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -131,7 +134,8 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmA
   const int tm = first_m + in_group % gsize, tn = in_group / gsize;
   const int m0 = tm * GBM, n0 = tn * GBN;
 
-  GemmTileLoader<C> xl, wl;
+  GemmTileLoader<C, C::kXPerWave> xl;
+  GemmTileLoader<C, C::kWPerWave> wl;
   xl.init(a.ldx, a.M - m0, wave, lane);
   wl.init(a.ldw, GBN, wave, lane);
   const char* xbase = reinterpret_cast<const char*>(a.x + (int64_t)m0 * a.ldx);
@@ -149,12 +153,16 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmA
   // the bias of this wave's columns, loaded before the k-loop: in the epilogue its
   // loads stood first on the critical path (1-1.3% of the launch)
   constexpr int kCols = C::TN * 32;              // this wave's columns (64 or 128)
+  constexpr bool kEarlyBias = C::TM < 5;         // (with five row blocks there is no register left)
   bf16x4 bias_r[C::TN][4];
+  auto load_bias = [&] {
 #pragma unroll
-  for (int nb = 0; nb < C::TN; ++nb)
+    for (int nb = 0; nb < C::TN; ++nb)
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
-      bias_r[nb][g] = *reinterpret_cast<const bf16x4*>(a.bias + n0 + wn * kCols + nb * 32 + 8 * g + 4 * hh);
+      for (int g = 0; g < 4; ++g)
+        bias_r[nb][g] = *reinterpret_cast<const bf16x4*>(a.bias + n0 + wn * kCols + nb * 32 + 8 * g + 4 * hh);
+  };
+  if constexpr (kEarlyBias) load_bias();
 
   f32x16 acc[C::TN][C::TM];
 #pragma unroll
@@ -172,15 +180,15 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmA
   };
   auto copy_one = [&](int slot, int kt, int i) {
     const int64_t kb = (int64_t)kt * BK * 2;
-    if (i < C::kPerWave)
+    if (i < C::kXPerWave)
       xl.issue_one(xbase + kb, xs[slot], wave, i);
     else
-      wl.issue_one(wbase + kb, ws[slot], wave, i - C::kPerWave);
+      wl.issue_one(wbase + kb, ws[slot], wave, i - C::kXPerWave);
   };
   constexpr int KS = BK / 16;             // MFMA k-steps per tile
   constexpr int NF = C::TN + C::TM;       // fragment reads per k-step
   constexpr int NM = C::TN * C::TM;       // MFMAs per k-step
-  constexpr int NC = 2 * C::kPerWave;     // copies per tile and wave
+  constexpr int NC = C::kXPerWave + C::kWPerWave;  // copies per tile and wave
   constexpr int SPLIT = NM - NF;          // MFMAs of the last k-step before the barrier
   static_assert(KS % 2 == 0 && NF <= NM, "schedule");
 
@@ -188,13 +196,15 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmA
 
   // One tile of k.  Program order is fixed MFMA by MFMA (a scheduling barrier after
   // each): after MFMA m of k-step ks comes fragment read m of k-step ks + 1 (the reads
-  // are in flight behind the MFMAs that follow) and, in k-step 0, copy m of the next
-  // tile into the other slot.  The last k-step splits around the barrier that publishes
-  // the next tile: NM - NF MFMAs, the copies' wait and the barrier, then NF MFMAs, each
-  // followed by a read of the next tile's first k-step.
-  auto tile = [&](int kt, auto has_next_c) {
-    constexpr bool has_next = decltype(has_next_c)::value;
-    const int slot = kt & 1, nslot = slot ^ 1;
+  // are in flight behind the MFMAs that follow) and, in k-step 0, copy m of the tile
+  // SLOTS - 1 ahead into the slot that the tile before this one left.  The last k-step
+  // splits around the barrier that publishes the next tile: NM - NF MFMAs, the wait for
+  // that tile's copies (those of later tiles stay in flight) and the barrier, then NF
+  // MFMAs, each followed by a read of the next tile's first k-step.
+  int slot = 0;                       // of tile kt
+  auto tile = [&](int kt, auto next_c, auto copy_c) {
+    constexpr bool has_next = decltype(next_c)::value, has_copy = decltype(copy_c)::value;
+    const int nslot = slot == SLOTS - 1 ? 0 : slot + 1, cslot = slot == 0 ? SLOTS - 1 : slot - 1;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const int cur = ks & 1, nxt = cur ^ 1;
@@ -202,7 +212,10 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmA
       for (int m = 0; m < NM; ++m) {
         if (ks == KS - 1 && m == SPLIT) {
           // every wave's copies of the next tile landed, every read of this slot returned
-          asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+          if constexpr (has_copy && SLOTS > 2)
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "i"((SLOTS - 2) * NC) : "memory");
+          else
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
           __builtin_amdgcn_sched_barrier(0);
         }
         const int nb = m / C::TM, mb = m % C::TM;
@@ -212,23 +225,31 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmA
         } else if (has_next && m >= SPLIT) {
           read_frag(nslot, 0, m - SPLIT, wf[nxt], xf[nxt]);
         }
-        if (has_next && ks == 0 && m < NC) copy_one(nslot, kt + 1, m);
+        if (has_copy && ks == 0 && m < NC) copy_one(cslot, kt + SLOTS - 1, m);
         __builtin_amdgcn_sched_barrier(0);
       }
-      if (has_next && ks == 0) {
+      if (has_copy && ks == 0) {
 #pragma unroll
-        for (int i = NM; i < NC; ++i) copy_one(nslot, kt + 1, i);
+        for (int i = NM; i < NC; ++i) copy_one(cslot, kt + SLOTS - 1, i);
       }
     }
+    slot = nslot;
   };
 
-  for (int i = 0; i < NC; ++i) copy_one(0, 0, i);
+  for (int t = 0; t < SLOTS - 1 && t < kt_count; ++t)
+    for (int i = 0; i < NC; ++i) copy_one(t, t, i);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < NF; ++i) read_frag(0, 0, i, wf[0], xf[0]);
-  for (int kt = 0; kt + 1 < kt_count; ++kt) tile(kt, std::integral_constant<bool, true>{});
-  tile(kt_count - 1, std::integral_constant<bool, false>{});
+  using yes = std::integral_constant<bool, true>;
+  using no = std::integral_constant<bool, false>;
+  int kt = 0;
+  for (; kt + SLOTS - 1 < kt_count; ++kt) tile(kt, yes{}, yes{});
+  if constexpr (SLOTS > 2)
+    for (; kt + 1 < kt_count; ++kt) tile(kt, yes{}, no{});
+  tile(kt, no{}, no{});
+  if constexpr (!kEarlyBias) load_bias();
   __syncthreads();   // every wave is done with the last stage before the output staging
 
   // Epilogue, one 32-row block at a time: bias, bf16 rounding, the sums of squares over
@@ -277,16 +298,51 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmA
   }
 }
 
+// Tile heights: the x rows of a workgroup's tile, and what a round of such tiles (one
+// workgroup per CU) takes at K = 3072, in us, from 1 to 9 rounds at N = 9216.
+constexpr struct { int rows; float round_us; } kTiles[] = {{320, 89.f}, {256, 72.f}, {192, 60.f}, {128, 42.f}};
+
+// The height whose rounds take least: a round that is mostly empty costs what a full one
+// costs, so between two heights the number of rounds decides.  N = 9216, us with 256 rows
+// and as chosen here:
+//   M 256   58.0 -> 34.0 (128)    M 1080  66.9 -> 58 (192)      M 2160  137 -> 95 (320)
+//   M 4114   214 -> 179 (320)     M 8228   376 -> 357 (320)     M 15708  684 (256)
+// The round times scale with K alike, so the choice depends on M and N alone.
+int tile_rows(int M, int N, int cus) {
+  int best = 0;
+  float best_us = 0.f;
+  for (const auto& t : kTiles) {
+    const int64_t tiles = ((int64_t)M + t.rows - 1) / t.rows * (N / GBN);
+    const float us = (float)((tiles + cus - 1) / cus) * t.round_us;
+    if (best == 0 || us < best_us) {
+      best = t.rows;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
+template <int GBM, int SLOTS>
+int launch_rows(const GemmArgs& a, hipStream_t s) {
+  const int64_t tiles = ((int64_t)a.M + GBM - 1) / GBM * (a.N / GBN);
+  if (tiles > 0x7fffffff) return set_error(2, "gemm: %lld tiles too many", (long long)tiles);
+  hipLaunchKernelGGL((gemm_rowsq_kernel<kGemmWM, kGemmWN, kGemmBK, GBM, SLOTS>), dim3((unsigned)tiles),
+                     dim3(64 * kGemmWM * kGemmWN), 0, s, a);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : set_error(4, "gemm launch: %s", hipGetErrorString(e));
+}
+
 }  // namespace
 
 int launch_gemm_rowsq(const GemmArgs& a, hipStream_t s) {
   if (a.M == 0) return 0;
-  const int64_t tiles = (int64_t)((a.M + GBM - 1) / GBM) * (a.N / GBN);
-  if (tiles > 0x7fffffff) return set_error(2, "gemm: %lld tiles too many", (long long)tiles);
-  hipLaunchKernelGGL((gemm_rowsq_kernel<kGemmWM, kGemmWN, kGemmBK>), dim3((unsigned)tiles),
-                     dim3(64 * kGemmWM * kGemmWN), 0, s, a);
-  const hipError_t e = hipGetLastError();
-  return e == hipSuccess ? 0 : set_error(4, "gemm launch: %s", hipGetErrorString(e));
+  // as many slots as the 160 KB of LDS hold
+  switch (tile_rows(a.M, a.N, device_cu_count())) {
+    case 320: return launch_rows<320, 2>(a, s);
+    case 256: return launch_rows<256, 2>(a, s);
+    case 192: return launch_rows<192, 2>(a, s);
+    default: return launch_rows<128, 3>(a, s);
+  }
 }
 
 }  // namespace wan
