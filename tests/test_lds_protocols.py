@@ -176,3 +176,24 @@ def test_ring4_planted_mistakes_are_caught(mistake):
     with pytest.raises(AssertionError):
         for n in range(1, 20):
             _check_protocol(n, **{mistake: True})
+
+
+@pytest.mark.parametrize("n", list(range(1, 40)) + [123])
+def test_wave_without_rows_keeps_the_protocol(n):
+    """A wave whose query rows all lie past Lq issues the same copies between the same barriers
+    as the others, without reading any: its own loop over the tiles, against theirs."""
+    K, V = lambda t: ("k", t % 4), lambda t: ("v", t % 4)
+    ops = [("issue", K(0), ("K", 0)), ("issue", V(0), ("V", 0)), ("wait",), ("bar",)]
+    if n > 1:
+        ops += [("issue", K(1), ("K", 1)), ("issue", V(1), ("V", 1))]
+    if n > 2:
+        ops += [("issue", K(2), ("K", 2))]
+    ops += [("wait",), ("bar",)]
+    for t in range(n - 1):
+        if t % 2 == 0:
+            ops += [("issue", K(i), ("K", i)) for i in (t + 3, t + 4) if i < n]
+            ops += [("issue", V(i), ("V", i)) for i in (t + 2, t + 3) if i < n]
+        else:
+            ops += [("wait",), ("bar",)]
+    ops.append(("bar",))
+    assert ops == [op for op in _ring4_ops(n) if op[0] in ("issue", "wait", "bar")]
