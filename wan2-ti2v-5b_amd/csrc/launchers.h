@@ -6,6 +6,24 @@
 
 namespace wan {
 
+// The sum of v over the W waves that work on one token row; `slot` names a sum of its own
+// where a kernel forms several (W = 1: the wave alone, no barrier).
+template <int W>
+__device__ __forceinline__ float row_sum(float v, int slot) {
+  v = wave_sum(v);
+  if constexpr (W == 1) {
+    return v;
+  } else {
+    __shared__ float part[2][W];
+    if ((threadIdx.x & 63) == 0) part[slot][threadIdx.x >> 6] = v;
+    __syncthreads();
+    float t = part[slot][0];
+#pragma unroll
+    for (int i = 1; i < W; ++i) t += part[slot][i];
+    return t;
+  }
+}
+
 struct PrepArgs {
   Tensor4 x;            // input rows [B, L, H, 128]
   int B, L, H;

@@ -15,12 +15,9 @@ namespace {
 
 constexpr int kMaxChunksPerLane = 16;  // supports H*128 <= 8192 channels per token
 
-// Rotate interleaved pairs of 8 consecutive channels d0..d0+7 of one token.
-__device__ __forceinline__ void rope8(float u[8], const float* cos_row,
-                                      const float* sin_row, int d0) {
+// Rotate interleaved pairs of 8 consecutive channels of one token by their four angles.
+__device__ __forceinline__ void rope8(float u[8], const f32x4 c, const f32x4 s) {
 #pragma clang fp contract(off)
-  const f32x4 c = *reinterpret_cast<const f32x4*>(cos_row + d0 / 2);
-  const f32x4 s = *reinterpret_cast<const f32x4*>(sin_row + d0 / 2);
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const float xr = u[2 * j], xi = u[2 * j + 1];
@@ -33,41 +30,64 @@ __device__ __forceinline__ void rope8(float u[8], const float* cos_row,
   }
 }
 
-// One wave per token row: sum of squares over all H*128 channels, then
-// optionally the normalised (and rotated) row.  NCH: 8-channel chunks per lane
-// (H*16 <= 64*NCH), so the row's loads are issued unconditionally together.  The
-// rows are read once here: non-temporal loads (4% faster alone at B=2, L=7854 than
-// plain ones, ~2 us a launch, below what a whole block forward resolves; the written
-// rows stay cacheable, the attention kernel reads them next).
-template <int NCH>
+// Sum of squares over all H*128 channels of a token row, then optionally the normalised (and
+// rotated) row.  W waves work on a row, each lane on NCH chunks of 8 channels (H*16 <= 64 W NCH):
+//   W = 1   four rows a block, the whole row in a wave's registers: for many rows, where the
+//           loads in flight of all the waves cover the latency;
+//   W > 1   one row a block, one chunk a lane: for few rows, where one wave's chain of loads,
+//           48 channels of arithmetic a lane and stores is what a launch takes.  Norm +
+//           rotation of 3072 channels, us: 1080 rows 7.9 -> 5.0, 2160 rows 11.5 -> 8.1.
+// All loads go out before the sum is formed.
+// NT: non-temporal loads of x, for rows that are not read again here and that together with
+// the rows written exceed what the 256 MB cache in front of the memory keeps from their writer
+// (15708 rows of norm + rotation 41.0 -> 39.4 us; 8228 rows 21.4 -> 25.6).  Never for
+// statistics alone: the attention kernel reads those rows next (norm + cross-attention,
+// batch 2: 7854 rows 137 us with non-temporal loads, 133 without; 1080 rows 25.8, 24.7).
+template <int NCH, int W, bool NT>
 __device__ __forceinline__ void rms_prep_rows(const PrepArgs& a, int block) {
-  const int lane = threadIdx.x & 63;
-  const int tok = block * 4 + (threadIdx.x >> 6);
+  const int t = W == 1 ? threadIdx.x & 63 : threadIdx.x;
+  const int tok = W == 1 ? block * 4 + (threadIdx.x >> 6) : block;
   if (tok >= a.B * a.L) return;
   const int b = tok / a.L, l = tok - b * a.L;
   const int nchunks = a.H * 16;
   const bf16* row = a.x.ptr + b * a.x.sb + (int64_t)l * a.x.st;
+  const bool want = a.out != nullptr;
 
-  bf16x8 xv[NCH];
+  bf16x8 xv[NCH], gv[NCH];
   float ss = 0.f;
-  if (a.sumsq != nullptr) {
-    // the projection GEMM's partial sums (one per lane, then the wave's sum); the row
-    // itself is read only when the normalised row is wanted
-    if (lane < a.sumsq_parts) ss = a.sumsq[(int64_t)(a.sumsq_first + lane) * (a.B * a.L) + tok];
-    if (a.out != nullptr) {
+  // with the projection GEMM's partial sums the row is read only when it is to be normalised
+  if (want || a.sumsq == nullptr) {
 #pragma unroll
-      for (int i = 0; i < NCH; ++i) {
-        const int c = lane + 64 * i;
-        if (c < nchunks) xv[i] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(row + (c >> 4) * a.x.sh + (c & 15) * 8));
+    for (int i = 0; i < NCH; ++i) {
+      const int c = t + 64 * W * i;
+      if (c < nchunks) {
+        const bf16x8* p = reinterpret_cast<const bf16x8*>(row + (c >> 4) * a.x.sh + (c & 15) * 8);
+        xv[i] = NT ? __builtin_nontemporal_load(p) : *p;
       }
     }
+  }
+  // the channel pairs of a lane's chunks are the same in every head: 64 W is a multiple of 16
+  const int d0 = (t & 15) * 8;
+  f32x4 cs = {}, sn = {};
+  if (want) {
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int c = t + 64 * W * i;
+      if (c < nchunks) gv[i] = *reinterpret_cast<const bf16x8*>(a.gamma + 8 * c);
+    }
+    if (a.cos != nullptr) {
+      cs = *reinterpret_cast<const f32x4*>(a.cos + (int64_t)l * kRopePairs + d0 / 2);
+      sn = *reinterpret_cast<const f32x4*>(a.sin + (int64_t)l * kRopePairs + d0 / 2);
+    }
+  }
+  if (a.sumsq != nullptr) {
+    const int lane = threadIdx.x & 63;   // one partial sum a lane, in every wave of the row
+    if (lane < a.sumsq_parts) ss = a.sumsq[(int64_t)(a.sumsq_first + lane) * (a.B * a.L) + tok];
+    ss = wave_sum(ss);
   } else {
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
-      const int c = lane + 64 * i;
-      if (c < nchunks) {
-        const int h = c >> 4, d0 = (c & 15) * 8;
-        xv[i] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(row + h * a.x.sh + d0));
+      if (t + 64 * W * i < nchunks) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const float f = (float)xv[i][j];
@@ -75,49 +95,45 @@ __device__ __forceinline__ void rms_prep_rows(const PrepArgs& a, int block) {
         }
       }
     }
+    ss = row_sum<W>(ss, 0);
   }
-  ss = wave_sum(ss);
   const float inv = 1.0f / sqrtf(ss / (float)(a.H * kHeadDim) + a.eps);
-  if (a.inv_rms != nullptr && lane == 0) a.inv_rms[tok] = inv;
-  if (a.out == nullptr) return;
+  if (a.inv_rms != nullptr && t == 0) a.inv_rms[tok] = inv;
+  if (!want) return;
 
-  const float* cos_row = a.cos ? a.cos + (int64_t)l * kRopePairs : nullptr;
-  const float* sin_row = a.sin ? a.sin + (int64_t)l * kRopePairs : nullptr;
   bf16* orow = a.out + (int64_t)tok * a.H * kHeadDim;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
-    const int c = lane + 64 * i;
+    const int c = t + 64 * W * i;
     if (c < nchunks) {
-      const int h = c >> 4, d0 = (c & 15) * 8;
-      const bf16x8 g = *reinterpret_cast<const bf16x8*>(a.gamma + h * kHeadDim + d0);
       float u[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const bf16 t = (bf16)((float)xv[i][j] * inv);
-        u[j] = (float)(bf16)((float)t * (float)g[j]);
+        const bf16 n = (bf16)((float)xv[i][j] * inv);
+        u[j] = (float)(bf16)((float)n * (float)gv[i][j]);
       }
-      if (cos_row) rope8(u, cos_row, sin_row, d0);
+      if (a.cos != nullptr) rope8(u, cs, sn);
       bf16x8 r;
 #pragma unroll
       for (int j = 0; j < 8; ++j) r[j] = (bf16)u[j];
-      *reinterpret_cast<bf16x8*>(orow + h * kHeadDim + d0) = r;
+      *reinterpret_cast<bf16x8*>(orow + 8 * c) = r;
     }
   }
 }
 
-template <int NCH>
-__global__ __launch_bounds__(256) void rms_prep_kernel(const PrepArgs a) {
-  rms_prep_rows<NCH>(a, blockIdx.x);
+template <int NCH, int W, bool NT>
+__global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void rms_prep_kernel(const PrepArgs a) {
+  rms_prep_rows<NCH, W, NT>(a, blockIdx.x);
 }
 
 // Two independent tasks (the q statistics and the k norm + rotation of one
 // self-attention call) in one launch: blocks [0, blocks0) run a0, the rest a1.
-template <int NCH>
-__global__ __launch_bounds__(256) void rms_prep2_kernel(const PrepArgs a0, const PrepArgs a1, int blocks0) {
-  if ((int)blockIdx.x < blocks0) rms_prep_rows<NCH>(a0, blockIdx.x);
-  else rms_prep_rows<NCH>(a1, blockIdx.x - blocks0);
+template <int NCH, int W, bool NT>
+__global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void rms_prep2_kernel(const PrepArgs a0, const PrepArgs a1,
+                                                                         int blocks0) {
+  if ((int)blockIdx.x < blocks0) rms_prep_rows<NCH, W, false>(a0, blockIdx.x);
+  else rms_prep_rows<NCH, W, NT>(a1, blockIdx.x - blocks0);
 }
-
 
 // One thread per 8 channels: out = rope(x), the _rope semantics on its own.
 __global__ __launch_bounds__(256) void rope_kernel(const RopeArgs a) {
@@ -135,48 +151,70 @@ __global__ __launch_bounds__(256) void rope_kernel(const RopeArgs a) {
   float u[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) u[j] = (float)x[j];
-  rope8(u, a.cos + (int64_t)l * kRopePairs, a.sin + (int64_t)l * kRopePairs, d0);
+  rope8(u, *reinterpret_cast<const f32x4*>(a.cos + (int64_t)l * kRopePairs + d0 / 2),
+        *reinterpret_cast<const f32x4*>(a.sin + (int64_t)l * kRopePairs + d0 / 2));
   bf16x8 r;
 #pragma unroll
   for (int j = 0; j < 8; ++j) r[j] = (bf16)u[j];
   *reinterpret_cast<bf16x8*>(a.out + chunk * 8) = r;
 }
 
-}  // namespace
+// Up to this many rows in a launch a row is a block's (W > 1).  Statistics alone: cross-
+// attention at 748 rows 19.4 -> 18.1 us, at 2160 24.7 -> 25.1.  With normalised rows: norm +
+// rotation at 2160 rows 10.2 -> 8.1, at 4488 13.7 -> 13.2, but the self-attention after it
+// 152 -> 155 us there (q and k, 8976 rows) and 48.0 -> 48.1 at 4320 rows.
+constexpr int kFewRowsStats = 2048, kFewRowsNorm = 4096;
+// Rows read and written beyond this many bytes are read with non-temporal loads.
+constexpr int64_t kStreamBytes = int64_t(128) << 20;
 
-int launch_rms_prep(const PrepArgs& a, hipStream_t s) {
-  const int rows = a.B * a.L;
-  if (rows == 0) return 0;
-  const int nch = a.H * 16;
-  if (nch > 64 * kMaxChunksPerLane) return set_error(2, "rms_prep: H*128=%d channels exceeds 8192", a.H * 128);
-  const dim3 grid((rows + 3) / 4), block(256);
-  if (nch <= 64) hipLaunchKernelGGL(rms_prep_kernel<1>, grid, block, 0, s, a);
-  else if (nch <= 128) hipLaunchKernelGGL(rms_prep_kernel<2>, grid, block, 0, s, a);
-  else if (nch <= 256) hipLaunchKernelGGL(rms_prep_kernel<4>, grid, block, 0, s, a);
-  else if (nch <= 384) hipLaunchKernelGGL(rms_prep_kernel<6>, grid, block, 0, s, a);
-  else if (nch <= 512) hipLaunchKernelGGL(rms_prep_kernel<8>, grid, block, 0, s, a);
-  else hipLaunchKernelGGL(rms_prep_kernel<16>, grid, block, 0, s, a);
+// Launches `a0` alone (a1 null) or both tasks.
+template <int NCH, int W, bool NT>
+int launch_prep(const PrepArgs& a0, const PrepArgs* a1, hipStream_t s) {
+  constexpr int R = W == 1 ? 4 : 1;   // rows per block
+  const dim3 block(W == 1 ? 256 : 64 * W);
+  const int blocks0 = (a0.B * a0.L + R - 1) / R;
+  if (a1 == nullptr)
+    hipLaunchKernelGGL((rms_prep_kernel<NCH, W, NT>), dim3(blocks0), block, 0, s, a0);
+  else
+    hipLaunchKernelGGL((rms_prep2_kernel<NCH, W, NT>), dim3(blocks0 + (a1->B * a1->L + R - 1) / R), block, 0, s,
+                       a0, *a1, blocks0);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : set_error(4, "rms_prep launch: %s", hipGetErrorString(e));
 }
 
-int launch_rms_prep2(const PrepArgs& a0, const PrepArgs& a1, hipStream_t s) {
-  if (a0.H != a1.H) return set_error(1, "rms_prep: the paired tasks differ in heads");
-  const int rows0 = a0.B * a0.L, rows1 = a1.B * a1.L;
-  if (rows0 == 0) return launch_rms_prep(a1, s);
-  if (rows1 == 0) return launch_rms_prep(a0, s);
+template <int N>
+int launch_prep_n(const PrepArgs& a0, const PrepArgs* a1, hipStream_t s) {
+  const int64_t rows = (int64_t)a0.B * a0.L + (a1 != nullptr ? (int64_t)a1->B * a1->L : 0);
+  const PrepArgs& last = a1 != nullptr ? *a1 : a0;   // the task that may write rows
+  if (rows <= (last.out != nullptr ? kFewRowsNorm : kFewRowsStats)) return launch_prep<1, N, false>(a0, a1, s);
+  if (last.out != nullptr && (int64_t)last.B * last.L * last.H * (kHeadDim * 4) > kStreamBytes)
+    return launch_prep<N, 1, true>(a0, a1, s);
+  return launch_prep<N, 1, false>(a0, a1, s);
+}
+
+int launch_prep_any(const PrepArgs& a0, const PrepArgs* a1, hipStream_t s) {
   const int nch = a0.H * 16;
   if (nch > 64 * kMaxChunksPerLane) return set_error(2, "rms_prep: H*128=%d channels exceeds 8192", a0.H * 128);
-  const int blocks0 = (rows0 + 3) / 4;
-  const dim3 grid(blocks0 + (rows1 + 3) / 4), block(256);
-  if (nch <= 64) hipLaunchKernelGGL(rms_prep2_kernel<1>, grid, block, 0, s, a0, a1, blocks0);
-  else if (nch <= 128) hipLaunchKernelGGL(rms_prep2_kernel<2>, grid, block, 0, s, a0, a1, blocks0);
-  else if (nch <= 256) hipLaunchKernelGGL(rms_prep2_kernel<4>, grid, block, 0, s, a0, a1, blocks0);
-  else if (nch <= 384) hipLaunchKernelGGL(rms_prep2_kernel<6>, grid, block, 0, s, a0, a1, blocks0);
-  else if (nch <= 512) hipLaunchKernelGGL(rms_prep2_kernel<8>, grid, block, 0, s, a0, a1, blocks0);
-  else hipLaunchKernelGGL(rms_prep2_kernel<16>, grid, block, 0, s, a0, a1, blocks0);
-  const hipError_t e = hipGetLastError();
-  return e == hipSuccess ? 0 : set_error(4, "rms_prep launch: %s", hipGetErrorString(e));
+  if (nch <= 64) return launch_prep_n<1>(a0, a1, s);
+  if (nch <= 128) return launch_prep_n<2>(a0, a1, s);
+  if (nch <= 256) return launch_prep_n<4>(a0, a1, s);
+  if (nch <= 384) return launch_prep_n<6>(a0, a1, s);
+  if (nch <= 512) return launch_prep_n<8>(a0, a1, s);
+  return launch_prep_n<16>(a0, a1, s);
+}
+
+}  // namespace
+
+int launch_rms_prep(const PrepArgs& a, hipStream_t s) {
+  if (a.B * a.L == 0) return 0;
+  return launch_prep_any(a, nullptr, s);
+}
+
+int launch_rms_prep2(const PrepArgs& a0, const PrepArgs& a1, hipStream_t s) {
+  if (a0.H != a1.H) return set_error(1, "rms_prep: the paired tasks differ in heads");
+  if (a0.B * a0.L == 0) return launch_rms_prep(a1, s);
+  if (a1.B * a1.L == 0) return launch_rms_prep(a0, s);
+  return launch_prep_any(a0, &a1, s);
 }
 
 int launch_rope(const RopeArgs& a, hipStream_t s) {
