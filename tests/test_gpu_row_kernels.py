@@ -1,5 +1,5 @@
-"""GPU: both forms of the token-row kernels (a row per wave, a row per block) at the row counts
-and channel counts where the launchers change between them and where a lane's chunks end.
+"""GPU: the forms of the token-row kernels (waves a row, chunks of 8 channels a lane) at the row
+counts and channel counts where the launchers change between them and where a lane's chunks end.
 
 The forms sum a row's squares in different orders, which moves a bf16 value of the normalised
 row across a rounding boundary now and then."""
@@ -21,7 +21,7 @@ def _inv64(x, eps):
 
 
 @pytest.mark.parametrize("H", [1, 4, 5, 8, 9, 16, 24, 25, 32, 33, 64])     # 64 W NCH = H*16 and one head past it
-@pytest.mark.parametrize("rows", [1, 2047, 2048, 2049])
+@pytest.mark.parametrize("rows", [1, 1024, 1025])
 def test_statistics(W, H, rows):
     x = _bf((1, rows, H, D), H * rows, 2.0)
     inv = W.ops.rms_inv(x, 1e-6)
@@ -30,11 +30,11 @@ def test_statistics(W, H, rows):
     assert ((inv.double() - want).abs() <= want * (H * D + 8) * 2 ** -24).all()
 
 
-@pytest.mark.parametrize("H,rows", [(24, 4095), (24, 4096), (24, 4097), (5, 3), (33, 4097), (24, 10923), (24, 10924)])
+@pytest.mark.parametrize("H,rows", [(24, 1024), (24, 1025), (5, 3), (5, 1025), (33, 1025), (24, 10922), (24, 10923)])
 @pytest.mark.parametrize("rotate", [False, True])
 def test_normalised_rows(W, H, rows, rotate):
-    """Strided rows (a view of a wider projection); 4096 rows is where the form changes and
-    10923 (128 MB read and written) where the loads become non-temporal."""
+    """Strided rows (a view of a wider projection); 1024 rows is where the form changes and
+    10923 (128 MB read and written) where the stores become plain ones."""
     x = _bf((1, rows, 2 * H * D), rows, 2.0)[..., H * D:].view(1, rows, H, D)
     g = 1 + _bf((H * D,), 7).abs()
     ang = torch.rand(rows, 64, device=DEV) * 6
@@ -54,3 +54,18 @@ def test_normalised_rows(W, H, rows, rotate):
     # pair is rounded once more, by 2^-9 of its length and 2^-8 at most
     assert ((got - u).abs() <= size * (2 ** -6 + 2 ** -8)).all()
     assert float(((got - u).abs() > size * (2 ** -8 if rotate else 0)).double().mean()) < 1e-2
+
+
+@pytest.mark.parametrize("C", [8, 512, 520, 1024, 1032, 2048, 2056, 3072, 3080, 4096, 4104, 8192])
+@pytest.mark.parametrize("rows", [1, 6])
+def test_adaln_channels(W, C, rows):
+    """Gated residual, LayerNorm and modulation where a lane's chunks or a row's waves end."""
+    x, y, e = _bf((1, rows, C), C), _bf((1, rows, C), C + 1), _bf((1, 6, C), C + 2, 0.5)
+    r, h = W.ops.adaln(x, y, e, 1, gate_idx=2, shift_idx=0, scale_idx=1)
+    assert torch.equal(r, x + y * e[:, 2])
+    d = r.double()
+    n = (d - d.mean(-1, keepdim=True)) * (d.var(-1, unbiased=False, keepdim=True) + 1e-6).rsqrt()
+    s1, sh = (1 + e[:, 1]).double(), e[:, 0].double()
+    # roundings of the norm (2^-9 and the sums' order), of its product (2^-9) and of the result
+    size = (n * s1).abs()
+    assert ((h.double() - (n * s1 + sh)).abs() <= size * (2 ** -7 + 2 ** -9) + (size + sh.abs()) * 2 ** -8 + 1e-6).all()

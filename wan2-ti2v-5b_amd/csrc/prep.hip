@@ -31,18 +31,18 @@ __device__ __forceinline__ void rope8(float u[8], const f32x4 c, const f32x4 s) 
 }
 
 // Sum of squares over all H*128 channels of a token row, then optionally the normalised (and
-// rotated) row.  W waves work on a row, each lane on NCH chunks of 8 channels (H*16 <= 64 W NCH):
-//   W = 1   four rows a block, the whole row in a wave's registers: for many rows, where the
-//           loads in flight of all the waves cover the latency;
-//   W > 1   one row a block, one chunk a lane: for few rows, where one wave's chain of loads,
-//           48 channels of arithmetic a lane and stores is what a launch takes.  Norm +
-//           rotation of 3072 channels, us: 1080 rows 7.9 -> 5.0, 2160 rows 11.5 -> 8.1.
+// rotated) row.  W waves work on a row, each lane on NCH chunks of 8 channels (H*16 <= 64 W NCH).
+// With W > 1 a block is one row, with W = 1 (up to 1024 channels) four.  A row in one wave was
+// latency bound: too few loads in flight a CU, and for few rows one wave's chain of loads, 48
+// channels of arithmetic a lane and stores was what the launch took.  At 3072 channels, us with
+// 1 / 3 / 6 waves a row (the kernels of a call as the launcher chooses now):
+//   norm + rotation   748 rows 6.1 / 5.2 / 4.7   2160 rows 10.3 / 8.4 / 8.8   15708 rows 41.9 / 36.6 / 47.1
+//   statistics        748 rows 4.1 / 3.4 / 3.4   2160 rows  5.4 / 5.0 / 5.9   15708 rows 20.2 / 17.6 / 26.7
 // All loads go out before the sum is formed.
-// NT: non-temporal loads of x, for rows that are not read again here and that together with
-// the rows written exceed what the 256 MB cache in front of the memory keeps from their writer
-// (15708 rows of norm + rotation 41.0 -> 39.4 us; 8228 rows 21.4 -> 25.6).  Never for
-// statistics alone: the attention kernel reads those rows next (norm + cross-attention,
-// batch 2: 7854 rows 137 us with non-temporal loads, 133 without; 1080 rows 25.8, 24.7).
+// NT: non-temporal stores of the normalised rows.  No XCD's L2 keeps them for the next kernel,
+// and the launch does not end with their write-back (norm + rotation 2160 rows 8.4 -> 7.0 us,
+// 8228 rows 22.0 -> 20.1); with more than the last-level cache takes of rows read and written
+// they cost (15708 rows 36.6 -> 38.9).
 template <int NCH, int W, bool NT>
 __device__ __forceinline__ void rms_prep_rows(const PrepArgs& a, int block) {
   const int t = W == 1 ? threadIdx.x & 63 : threadIdx.x;
@@ -60,10 +60,7 @@ __device__ __forceinline__ void rms_prep_rows(const PrepArgs& a, int block) {
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       const int c = t + 64 * W * i;
-      if (c < nchunks) {
-        const bf16x8* p = reinterpret_cast<const bf16x8*>(row + (c >> 4) * a.x.sh + (c & 15) * 8);
-        xv[i] = NT ? __builtin_nontemporal_load(p) : *p;
-      }
+      if (c < nchunks) xv[i] = *reinterpret_cast<const bf16x8*>(row + (c >> 4) * a.x.sh + (c & 15) * 8);
     }
   }
   // the channel pairs of a lane's chunks are the same in every head: 64 W is a multiple of 16
@@ -116,7 +113,9 @@ __device__ __forceinline__ void rms_prep_rows(const PrepArgs& a, int block) {
       bf16x8 r;
 #pragma unroll
       for (int j = 0; j < 8; ++j) r[j] = (bf16)u[j];
-      *reinterpret_cast<bf16x8*>(orow + 8 * c) = r;
+      bf16x8* op = reinterpret_cast<bf16x8*>(orow + 8 * c);
+      if (NT) __builtin_nontemporal_store(r, op);
+      else *op = r;
     }
   }
 }
@@ -131,7 +130,7 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void rms_prep_kernel(const P
 template <int NCH, int W, bool NT>
 __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void rms_prep2_kernel(const PrepArgs a0, const PrepArgs a1,
                                                                          int blocks0) {
-  if ((int)blockIdx.x < blocks0) rms_prep_rows<NCH, W, false>(a0, blockIdx.x);
+  if ((int)blockIdx.x < blocks0) rms_prep_rows<NCH, W, NT>(a0, blockIdx.x);
   else rms_prep_rows<NCH, W, NT>(a1, blockIdx.x - blocks0);
 }
 
@@ -159,12 +158,9 @@ __global__ __launch_bounds__(256) void rope_kernel(const RopeArgs a) {
   *reinterpret_cast<bf16x8*>(a.out + chunk * 8) = r;
 }
 
-// Up to this many rows in a launch a row is a block's (W > 1).  Statistics alone: cross-
-// attention at 748 rows 19.4 -> 18.1 us, at 2160 24.7 -> 25.1.  With normalised rows: norm +
-// rotation at 2160 rows 10.2 -> 8.1, at 4488 13.7 -> 13.2, but the self-attention after it
-// 152 -> 155 us there (q and k, 8976 rows) and 48.0 -> 48.1 at 4320 rows.
-constexpr int kFewRowsStats = 2048, kFewRowsNorm = 4096;
-// Rows read and written beyond this many bytes are read with non-temporal loads.
+// Up to this many rows in a launch a lane has one chunk of 8 channels, beyond it two.
+constexpr int kFewRows = 1024;
+// Normalised rows leave with plain stores when rows read and written exceed this many bytes.
 constexpr int64_t kStreamBytes = int64_t(128) << 20;
 
 // Launches `a0` alone (a1 null) or both tasks.
@@ -182,14 +178,16 @@ int launch_prep(const PrepArgs& a0, const PrepArgs* a1, hipStream_t s) {
   return e == hipSuccess ? 0 : set_error(4, "rms_prep launch: %s", hipGetErrorString(e));
 }
 
+// N: chunks a lane when a row is one wave's.
 template <int N>
 int launch_prep_n(const PrepArgs& a0, const PrepArgs* a1, hipStream_t s) {
   const int64_t rows = (int64_t)a0.B * a0.L + (a1 != nullptr ? (int64_t)a1->B * a1->L : 0);
   const PrepArgs& last = a1 != nullptr ? *a1 : a0;   // the task that may write rows
-  if (rows <= (last.out != nullptr ? kFewRowsNorm : kFewRowsStats)) return launch_prep<1, N, false>(a0, a1, s);
-  if (last.out != nullptr && (int64_t)last.B * last.L * last.H * (kHeadDim * 4) > kStreamBytes)
-    return launch_prep<N, 1, true>(a0, a1, s);
-  return launch_prep<N, 1, false>(a0, a1, s);
+  if (rows <= kFewRows) return launch_prep<1, N, true>(a0, a1, s);
+  if constexpr (N == 1) return launch_prep<1, 1, true>(a0, a1, s);
+  else if ((int64_t)last.B * last.L * last.H * (kHeadDim * 4) > kStreamBytes)
+    return launch_prep<2, N / 2, false>(a0, a1, s);
+  else return launch_prep<2, N / 2, true>(a0, a1, s);
 }
 
 int launch_prep_any(const PrepArgs& a0, const PrepArgs* a1, hipStream_t s) {
