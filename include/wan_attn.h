@@ -271,6 +271,17 @@ int wan_qkv_proj_sumsq(const void* x, const void* w, const void* bias, void* out
                        int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int sq_cols,
                        void* stream);
 
+/*
+ * wan_qkv_proj_sumsq with scratch: where the tiles of the output leave half of the CUs or more
+ * idle in their last round, those are split over k and their fp32 sums joined through
+ * `workspace` (256-byte aligned, of wan_qkv_proj_workspace() bytes; 0: this size does not
+ * split).  With NULL or fewer bytes the call runs with what fits, or unsplit.
+ */
+size_t wan_qkv_proj_workspace(int M, int N, int K);
+int wan_qkv_proj_sumsq_ws(const void* x, const void* w, const void* bias, void* out, float* sumsq,
+                          int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int sq_cols,
+                          void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

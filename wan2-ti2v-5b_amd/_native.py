@@ -55,6 +55,8 @@ SIGNATURES = {
     "wan_adaln": (_I, [_P, _P, _P, _P, _I, _I, _I, _P, _I, _I, _I, _I, _P, _P, _F, _P]),
     "wan_adaln_ex": (_I, [_P, _P, _P, _P, _I, _I, _I, _P, _I, _I, _P, _I, _I, _I, _P, _P, _F, _P]),
     "wan_qkv_proj_sumsq": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _L, _L, _L, _I, _P]),
+    "wan_qkv_proj_workspace": (_SZ, [_I, _I, _I]),
+    "wan_qkv_proj_sumsq_ws": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _L, _L, _L, _I, _P, _SZ, _P]),
     "wan_rms_norm_qk_sumsq": (_I, [_T, _P, _I, _I, _I, _I, _P, _F, _P, _P, _P, _P, _P]),
 }
 

@@ -512,9 +512,13 @@ int wan_rope(wan_tensor x, void* out, int batch, int seqlen, int heads, int head
   return launch_rope(a, static_cast<hipStream_t>(stream));
 }
 
-int wan_qkv_proj_sumsq(const void* x, const void* w, const void* bias, void* out, float* sumsq,
-                       int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int sq_cols,
-                       void* stream) {
+size_t wan_qkv_proj_workspace(int M, int N, int K) {
+  return M > 0 && N > 0 && K > 0 && N % 256 == 0 && K % 64 == 0 ? gemm_split_bytes(M, N, K) : 0;
+}
+
+int wan_qkv_proj_sumsq_ws(const void* x, const void* w, const void* bias, void* out, float* sumsq,
+                          int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int sq_cols,
+                          void* workspace, size_t workspace_bytes, void* stream) {
   const char* fn = "wan_qkv_proj_sumsq";
   if (M < 0 || N <= 0 || K <= 0)
     return set_error(WAN_ERR_INVALID, "%s: bad sizes (M=%d N=%d K=%d)", fn, M, N, K);
@@ -537,7 +541,7 @@ int wan_qkv_proj_sumsq(const void* x, const void* w, const void* bias, void* out
   for (const void* p : ptrs)
     if (!aligned16(p))
       return set_error(WAN_ERR_INVALID, "%s: operands must be 16-byte aligned device pointers", fn);
-  GemmArgs a;
+  GemmArgs a{};
   a.x = static_cast<const bf16*>(x);
   a.w = static_cast<const bf16*>(w);
   a.bias = static_cast<const bf16*>(bias);
@@ -550,7 +554,17 @@ int wan_qkv_proj_sumsq(const void* x, const void* w, const void* bias, void* out
   a.ldw = ldw;
   a.ldo = ldo;
   a.sq_cols = sq_cols;
+  if (workspace != nullptr && reinterpret_cast<uintptr_t>(workspace) % kAlign)
+    return set_error(WAN_ERR_INVALID, "%s: workspace must be 256-byte aligned", fn);
+  a.part = static_cast<float*>(workspace);
+  a.part_bytes = workspace_bytes;
   return launch_gemm_rowsq(a, static_cast<hipStream_t>(stream));
+}
+
+int wan_qkv_proj_sumsq(const void* x, const void* w, const void* bias, void* out, float* sumsq,
+                       int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int sq_cols,
+                       void* stream) {
+  return wan_qkv_proj_sumsq_ws(x, w, bias, out, sumsq, M, N, K, ldx, ldw, ldo, sq_cols, nullptr, 0, stream);
 }
 
 int wan_adaln_ex(const void* x, const void* y, void* x_out, void* h_out, int batch, int seqlen,

@@ -112,7 +112,59 @@ struct GemmTileLoader {
   }
 };
 
-template <int WM, int WN, int BK, int GBM, int SLOTS>
+// First row and column of output tile `pid`: groups of kGroupM M-tiles, N-tiles within a group.
+__device__ __forceinline__ void tile_origin(const GemmArgs& a, int pid, int rows, int& m0, int& n0) {
+  const int mt_count = (a.M + rows - 1) / rows, nt_count = a.N / GBN;
+  const int per_group = kGroupM * nt_count;
+  const int group = pid / per_group, first_m = group * kGroupM;
+  const int gsize = min(mt_count - first_m, kGroupM);
+  const int in_group = pid - group * per_group;
+  m0 = (first_m + in_group % gsize) * rows;
+  n0 = in_group / gsize * GBN;
+}
+
+// A 32-row block of a wave's columns (64 TN / 2, from column ncol0): the sums of squares over
+// each 64 of them and the rounded rows, staged through this wave's LDS (row-major, chunk c of
+// row r at position c ^ (r % chunks)) and stored as whole row segments.  `value` gives the
+// lane's four values of row l32 from column 32 nb + 8 g + 4 hh of the block on.
+template <int TN, typename F>
+__device__ __forceinline__ void store_rows32(const GemmArgs& a, int row0, int ncol0, bf16* stage, int lane, F value) {
+  constexpr int kCols = TN * 32, kChunks = kCols / 8;
+  const int l32 = lane & 31, hh = lane >> 5;
+  float ss[TN / 2] = {};
+#pragma unroll
+  for (int nb = 0; nb < TN; ++nb) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const bf16x4 v = value(nb, g);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float f = (float)v[e];
+        ss[nb / 2] = fmaf(f, f, ss[nb / 2]);
+      }
+      const int c = 4 * nb + g;   // this lane's columns 8c + 4hh .. +3 of row l32
+      *reinterpret_cast<bf16x4*>(stage + l32 * kCols + ((c ^ (l32 % kChunks)) << 3) + 4 * hh) = v;
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < TN / 2; ++h) {
+    const float t = pair_sum(ss[h]);
+    if (ncol0 + 64 * h < a.sq_cols && hh == 0 && row0 + l32 < a.M)
+      a.sumsq[(int64_t)(ncol0 / 64 + h) * a.M + row0 + l32] = t;
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  constexpr int kRowsPerStore = 64 / kChunks;
+#pragma unroll
+  for (int j = 0; j < 32 / kRowsPerStore; ++j) {
+    const int r = kRowsPerStore * j + lane / kChunks, c = lane % kChunks;
+    const bf16x8 v = *reinterpret_cast<const bf16x8*>(stage + r * kCols + ((c ^ (r % kChunks)) << 3));
+    if (row0 + r < a.M)
+      __builtin_nontemporal_store(v, reinterpret_cast<bf16x8*>(a.out + (int64_t)(row0 + r) * a.ldo + ncol0 + 8 * c));
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+}
+
+template <int WM, int WN, int BK, int GBM, int SLOTS, bool SPLIT>
 __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmArgs a) {
   using C = GemmCfg<WM, WN, BK, GBM>;
   __shared__ __attribute__((aligned(1024))) bf16 xs[SLOTS][GBM * BK];
@@ -124,22 +176,29 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmA
   const int wm = wave % WM, wn = wave / WM;
   const int l32 = lane & 31, hh = lane >> 5;
 
-  // tile order: groups of kGroupM M-tiles, N-tiles within a group, each XCD a range
-  const int mt_count = (a.M + GBM - 1) / GBM, nt_count = a.N / GBN;
-  const int pid = xcd_remap(blockIdx.x, gridDim.x);
-  const int per_group = kGroupM * nt_count;
-  const int group = pid / per_group, first_m = group * kGroupM;
-  const int gsize = min(mt_count - first_m, kGroupM);
-  const int in_group = pid - group * per_group;
-  const int tm = first_m + in_group % gsize, tn = in_group / gsize;
-  const int m0 = tm * GBM, n0 = tn * GBN;
+  // Each XCD owns a contiguous range of the tiles, and of the split parts: those part by part,
+  // so that the tiles of one k range that run together on an XCD share x and w rows.
+  int pid, part = -1, kt_first = 0, kt_count = a.K / BK;
+  if (!SPLIT || (int)blockIdx.x < a.split_from) {
+    pid = xcd_remap(blockIdx.x, SPLIT ? a.split_from : gridDim.x);
+  } else {
+    const int n = gridDim.x - a.split_from, tiles = n / a.splits;
+    const int i = xcd_remap(blockIdx.x - a.split_from, n);
+    const int k = i / tiles, tile = i - k * tiles;
+    pid = a.split_from + tile;
+    part = tile * a.splits + k;
+    kt_first = (int)((int64_t)kt_count * k / a.splits);
+    kt_count = (int)((int64_t)kt_count * (k + 1) / a.splits) - kt_first;
+  }
+  int m0, n0;
+  tile_origin(a, pid, GBM, m0, n0);
 
   GemmTileLoader<C, C::kXPerWave> xl;
   GemmTileLoader<C, C::kWPerWave> wl;
   xl.init(a.ldx, a.M - m0, wave, lane);
   wl.init(a.ldw, GBN, wave, lane);
-  const char* xbase = reinterpret_cast<const char*>(a.x + (int64_t)m0 * a.ldx);
-  const char* wbase = reinterpret_cast<const char*>(a.w + (int64_t)n0 * a.ldw);
+  const char* xbase = reinterpret_cast<const char*>(a.x + (int64_t)m0 * a.ldx + kt_first * BK);
+  const char* wbase = reinterpret_cast<const char*>(a.w + (int64_t)n0 * a.ldw + kt_first * BK);
 
   // operand rows of this lane within the tiles; (row / kRps) % kCpr is the same for
   // every 32-row block
@@ -170,7 +229,6 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmA
 #pragma unroll
     for (int j = 0; j < C::TM; ++j) acc[i][j] = f32x16{};
 
-  const int kt_count = a.K / BK;
   auto read_frag = [&](int slot, int ks, int i, bf16x8 wf[C::TN], bf16x8 xf[C::TM]) {
     const int pos = ((2 * ks + hh) ^ sw) << 3;
     if (i < C::TN)
@@ -189,7 +247,7 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmA
   constexpr int NF = C::TN + C::TM;       // fragment reads per k-step
   constexpr int NM = C::TN * C::TM;       // MFMAs per k-step
   constexpr int NC = C::kXPerWave + C::kWPerWave;  // copies per tile and wave
-  constexpr int SPLIT = NM - NF;          // MFMAs of the last k-step before the barrier
+  constexpr int PRE = NM - NF;            // MFMAs of the last k-step before the barrier
   static_assert(KS % 2 == 0 && NF <= NM, "schedule");
 
   bf16x8 wf[2][C::TN], xf[2][C::TM];
@@ -210,7 +268,7 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmA
       const int cur = ks & 1, nxt = cur ^ 1;
 #pragma unroll
       for (int m = 0; m < NM; ++m) {
-        if (ks == KS - 1 && m == SPLIT) {
+        if (ks == KS - 1 && m == PRE) {
           // every wave's copies of the next tile landed, every read of this slot returned
           if constexpr (has_copy && SLOTS > 2)
             asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "i"((SLOTS - 2) * NC) : "memory");
@@ -222,8 +280,8 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmA
         acc[nb][mb] = mfma32(wf[cur][nb], xf[cur][mb], acc[nb][mb]);
         if (ks < KS - 1) {
           if (m < NF) read_frag(slot, ks + 1, m, wf[nxt], xf[nxt]);
-        } else if (has_next && m >= SPLIT) {
-          read_frag(nslot, 0, m - SPLIT, wf[nxt], xf[nxt]);
+        } else if (has_next && m >= PRE) {
+          read_frag(nslot, 0, m - PRE, wf[nxt], xf[nxt]);
         }
         if (has_copy && ks == 0 && m < NC) copy_one(cslot, kt + SLOTS - 1, m);
         __builtin_amdgcn_sched_barrier(0);
@@ -249,99 +307,151 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmA
   if constexpr (SLOTS > 2)
     for (; kt + 1 < kt_count; ++kt) tile(kt, yes{}, no{});
   tile(kt, no{}, no{});
+  if (SPLIT && part >= 0) {
+    // fp32, 64 lanes x 4 values a store: block (wave, mb, nb, g) of 1 KB
+    float* p = a.part + (int64_t)part * (GBM * GBN) + wave * (C::TM * C::TN * 1024) + lane * 4;
+#pragma unroll
+    for (int mb = 0; mb < C::TM; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < C::TN; ++nb)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          f32x4 v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = acc[nb][mb][4 * g + e];
+          *reinterpret_cast<f32x4*>(p + ((mb * C::TN + nb) * 4 + g) * 256) = v;
+        }
+    return;
+  }
   if constexpr (!kEarlyBias) load_bias();
   __syncthreads();   // every wave is done with the last stage before the output staging
 
-  // Epilogue, one 32-row block at a time: bias, bf16 rounding, the sums of squares over
-  // each 64 of this wave's columns, then the block staged through this wave's LDS
-  // (row-major, chunk c of row r at position c ^ (r % chunks)) and stored as whole row
-  // segments.
-  constexpr int kChunks = kCols / 8;
   bf16* stage = &xs[0][0] + wave * 32 * kCols;
-  const int ncol0 = n0 + wn * kCols;
 #pragma unroll
-  for (int mb = 0; mb < C::TM; ++mb) {
-    const int row0 = m0 + (wm * C::TM + mb) * 32;
-    float ss[C::TN / 2] = {};   // per 64 columns (two 32-column blocks)
+  for (int mb = 0; mb < C::TM; ++mb)
+    store_rows32<C::TN>(a, m0 + (wm * C::TM + mb) * 32, n0 + wn * kCols, stage, lane, [&](int nb, int g) {
+      bf16x4 v;
 #pragma unroll
-    for (int nb = 0; nb < C::TN; ++nb) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const bf16x4 b4 = bias_r[nb][g];
-        bf16x4 v;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          v[e] = (bf16)(acc[nb][mb][4 * g + e] + (float)b4[e]);
-          const float f = (float)v[e];
-          ss[nb / 2] = fmaf(f, f, ss[nb / 2]);
-        }
-        const int c = 4 * nb + g;   // this lane's columns 8c + 4hh .. +3 of row l32
-        *reinterpret_cast<bf16x4*>(stage + l32 * kCols + ((c ^ (l32 % kChunks)) << 3) + 4 * hh) = v;
-      }
-    }
-#pragma unroll
-    for (int h = 0; h < C::TN / 2; ++h) {
-      const float t = pair_sum(ss[h]);
-      if (ncol0 + 64 * h < a.sq_cols && hh == 0 && row0 + l32 < a.M)
-        a.sumsq[(int64_t)(ncol0 / 64 + h) * a.M + row0 + l32] = t;
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    constexpr int kRowsPerStore = 64 / kChunks;
-#pragma unroll
-    for (int j = 0; j < 32 / kRowsPerStore; ++j) {
-      const int r = kRowsPerStore * j + lane / kChunks, c = lane % kChunks;
-      const bf16x8 v = *reinterpret_cast<const bf16x8*>(stage + r * kCols + ((c ^ (r % kChunks)) << 3));
-      if (row0 + r < a.M)
-        __builtin_nontemporal_store(v, reinterpret_cast<bf16x8*>(a.out + (int64_t)(row0 + r) * a.ldo + ncol0 + 8 * c));
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  }
+      for (int e = 0; e < 4; ++e) v[e] = (bf16)(acc[nb][mb][4 * g + e] + (float)bias_r[nb][g][e]);
+      return v;
+    });
 }
 
-// Tile heights: the x rows of a workgroup's tile, and what a round of such tiles (one
-// workgroup per CU) takes at K = 3072, in us, from 1 to 9 rounds at N = 9216.
-constexpr struct { int rows; float round_us; } kTiles[] = {{320, 89.f}, {256, 72.f}, {192, 60.f}, {128, 42.f}};
+// The output of the split tiles: their parts summed in order, then the epilogue.  One wave per
+// 32 rows x 64 columns (a wave's 32-row block of the GEMM), four waves a workgroup.
+__global__ __launch_bounds__(256) void gemm_merge_kernel(const GemmArgs a, int rows) {
+  constexpr int TN = GBN / kGemmWN / 32;
+  __shared__ __attribute__((aligned(16))) bf16 stage[4][32 * TN * 32];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int hh = lane >> 5;
+  const int tm = rows / (32 * kGemmWM), per_tile = kGemmWM * kGemmWN * tm;
+  const int piece = blockIdx.x * 4 + wave;
+  const int tile = piece / per_tile, block = piece - tile * per_tile;
+  const int gw = block / tm, mb = block - gw * tm;      // the GEMM's wave and its 32-row block
+  int m0, n0;
+  tile_origin(a, a.split_from + tile, rows, m0, n0);
+  const int row0 = m0 + (gw % kGemmWM * tm + mb) * 32, ncol0 = n0 + gw / kGemmWM * (TN * 32);
+  if (row0 >= a.M) return;
 
-// The height whose rounds take least: a round that is mostly empty costs what a full one
-// costs, so between two heights the number of rounds decides.  N = 9216, us with 256 rows
-// and as chosen here:
-//   M 256   58.0 -> 34.0 (128)    M 1080  66.9 -> 58 (192)      M 2160  137 -> 95 (320)
-//   M 4114   214 -> 179 (320)     M 8228   376 -> 357 (320)     M 15708  684 (256)
-// The round times scale with K alike, so the choice depends on M and N alone.
-int tile_rows(int M, int N, int cus) {
-  int best = 0;
-  float best_us = 0.f;
+  const float* p = a.part + (int64_t)tile * a.splits * (rows * GBN) + block * (TN * 1024) + lane * 4;
+  f32x4 acc[TN][4];
+#pragma unroll
+  for (int i = 0; i < 4 * TN; ++i) acc[i / 4][i % 4] = *reinterpret_cast<const f32x4*>(p + i * 256);
+  for (int k = 1; k < a.splits; ++k) {
+    p += rows * GBN;
+#pragma unroll
+    for (int i = 0; i < 4 * TN; ++i) acc[i / 4][i % 4] += *reinterpret_cast<const f32x4*>(p + i * 256);
+  }
+  store_rows32<TN>(a, row0, ncol0, stage[wave], lane, [&](int nb, int g) {
+    const bf16x4 b = *reinterpret_cast<const bf16x4*>(a.bias + ncol0 + nb * 32 + 8 * g + 4 * hh);
+    bf16x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (bf16)(acc[nb][g][e] + (float)b[e]);
+    return v;
+  });
+}
+
+// Tile heights: the x rows of a workgroup's tile, and what a round of such tiles (one workgroup
+// per CU) takes, in us: per 64 of k, and besides (weights from memory, fitted over M 80 to 15708).
+constexpr struct { int rows; float k_us; } kTiles[] = {{320, 1.78f}, {256, 1.58f}, {192, 1.27f}, {128, 0.79f}};
+constexpr float kRoundUs = 10.f;
+// The merge launch, and the write and read of a part's row of 256 fp32 (plain stores: past the
+// L2s, non-temporally, the calls took 3-7 us longer).
+constexpr float kMergeUs = 4.f, kMergeRowUs = 2 * 256 * 4 / 8e6f;
+constexpr int kMaxSplits = 16, kMinSplitTiles = 4;
+
+// How a product is run: tiles of `rows` rows, the first `from` of them whole, the `rest` as
+// `splits` parts over k each.
+struct GemmPlan {
+  int rows, from, rest, splits;
+  float us;
+};
+
+// The plan whose rounds take least, with up to `scratch` bytes for the parts.  A round that is
+// mostly empty costs what a full one costs, so between two heights the number of rounds decides,
+// and where a last (or only) round leaves half of the CUs or more idle, its tiles may be split
+// over k: the parts' fp32 sums cost a merge launch and their way through memory.  us, tiles of
+// 256 rows alone / the best height / as chosen here:
+//   N 9216, K 3072:   M 80  59 / 45 / 28   M 256  58 / 48 / 32   M 2160  137 / 104 / 104 (320 rows)
+//                     M 8228  376 / 374 / 374 (320)   M 15708  756 / 756 / 690 (320, a tail of 8 tiles)
+//   N 3072, K 14336:  M 80  - / 182 / 36   M 748  - / 178 / 82   M 1500  - / 173 / 132
+//                     M 2160  - / 187 / 173 (320 rows, three parts)   M 8228  - / 739 / 581
+GemmPlan gemm_plan(int M, int N, int K, int cus, size_t scratch) {
+  GemmPlan best{0, 0, 0, 1, 0.f};
+  const int kt = K / kGemmBK;
   for (const auto& t : kTiles) {
     const int64_t tiles = ((int64_t)M + t.rows - 1) / t.rows * (N / GBN);
-    const float us = (float)((tiles + cus - 1) / cus) * t.round_us;
-    if (best == 0 || us < best_us) {
-      best = t.rows;
-      best_us = us;
+    const int64_t full = tiles / cus;
+    const int rest = (int)(tiles % cus);
+    for (int n = 1; n == 1 || (rest > 0 && n <= kMaxSplits && rest * n <= cus && n * kMinSplitTiles <= kt); ++n) {
+      if (n > 1 && (size_t)rest * n * t.rows * GBN * sizeof(float) > scratch) break;
+      float us = full * (kt * t.k_us + kRoundUs);
+      if (rest > 0) us += (kt + n - 1) / n * t.k_us + kRoundUs;
+      if (n > 1) us += kMergeUs + (float)rest * n * t.rows * kMergeRowUs;
+      if (best.rows == 0 || us < best.us) best = {t.rows, n > 1 ? (int)(tiles - rest) : 0, n > 1 ? rest : 0, n, us};
     }
   }
   return best;
 }
 
+size_t plan_bytes(const GemmPlan& p) { return p.splits > 1 ? (size_t)p.rest * p.splits * p.rows * GBN * sizeof(float) : 0; }
+
 template <int GBM, int SLOTS>
-int launch_rows(const GemmArgs& a, hipStream_t s) {
+int launch_rows(const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
   const int64_t tiles = ((int64_t)a.M + GBM - 1) / GBM * (a.N / GBN);
   if (tiles > 0x7fffffff) return set_error(2, "gemm: %lld tiles too many", (long long)tiles);
-  hipLaunchKernelGGL((gemm_rowsq_kernel<kGemmWM, kGemmWN, kGemmBK, GBM, SLOTS>), dim3((unsigned)tiles),
-                     dim3(64 * kGemmWM * kGemmWN), 0, s, a);
+  const dim3 block(64 * kGemmWM * kGemmWN);
+  if (p.splits > 1) {
+    GemmArgs as = a;
+    as.split_from = p.from;
+    as.splits = p.splits;
+    hipLaunchKernelGGL((gemm_rowsq_kernel<kGemmWM, kGemmWN, kGemmBK, GBM, SLOTS, true>),
+                       dim3((unsigned)(p.from + p.rest * p.splits)), block, 0, s, as);
+    hipLaunchKernelGGL(gemm_merge_kernel, dim3((unsigned)(p.rest * (GBM / 32))), dim3(256), 0, s, as, GBM);
+  } else {
+    hipLaunchKernelGGL((gemm_rowsq_kernel<kGemmWM, kGemmWN, kGemmBK, GBM, SLOTS, false>), dim3((unsigned)tiles),
+                       block, 0, s, a);
+  }
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : set_error(4, "gemm launch: %s", hipGetErrorString(e));
 }
 
 }  // namespace
 
+size_t gemm_split_bytes(int M, int N, int K) {
+  if (M <= 0 || N < GBN || K < kGemmBK) return 0;
+  return plan_bytes(gemm_plan(M, N, K, device_cu_count(), SIZE_MAX));
+}
+
 int launch_gemm_rowsq(const GemmArgs& a, hipStream_t s) {
   if (a.M == 0) return 0;
+  GemmPlan p = gemm_plan(a.M, a.N, a.K, device_cu_count(), a.part != nullptr ? a.part_bytes : 0);
   // as many slots as the 160 KB of LDS hold
-  switch (tile_rows(a.M, a.N, device_cu_count())) {
-    case 320: return launch_rows<320, 2>(a, s);
-    case 256: return launch_rows<256, 2>(a, s);
-    case 192: return launch_rows<192, 2>(a, s);
-    default: return launch_rows<128, 3>(a, s);
+  switch (p.rows) {
+    case 320: return launch_rows<320, 2>(a, p, s);
+    case 256: return launch_rows<256, 2>(a, p, s);
+    case 192: return launch_rows<192, 2>(a, p, s);
+    default: return launch_rows<128, 3>(a, p, s);
   }
 }
 

@@ -80,7 +80,15 @@ struct GemmArgs {
   int M, N, K;
   int64_t ldx, ldw, ldo;
   int sq_cols;          // multiple of 64, <= N
+  // Split of the last round of tiles over k: scratch given by the caller (null: none), and what
+  // the launcher makes of it: tiles before split_from are whole, those from there on are
+  // `splits` workgroups each that leave their fp32 sums in `part`.
+  float* part;
+  size_t part_bytes;
+  int split_from, splits;
 };
+// Scratch bytes that a product of this size makes use of (0: it does not split).
+size_t gemm_split_bytes(int M, int N, int K);
 int launch_gemm_rowsq(const GemmArgs& a, hipStream_t s);
 
 }  // namespace wan

@@ -394,10 +394,13 @@ def qkv_proj_sumsq(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor,
     _check_rows(fn, "bias", bias, (Nn,), x.device)
     out = torch.empty((B, L, Nn), dtype=x.dtype, device=x.device)
     sumsq = torch.empty((max(sq_cols // 64, 1), B * L), dtype=torch.float32, device=x.device)
+    lib = N.lib()
     with torch.cuda.device(x.device):
-        N.check("wan_qkv_proj_sumsq", N.lib().wan_qkv_proj_sumsq(
+        n = lib.wan_qkv_proj_workspace(B * L, Nn, C)
+        ws = torch.empty(n, dtype=torch.uint8, device=x.device) if n else None
+        N.check("wan_qkv_proj_sumsq", lib.wan_qkv_proj_sumsq_ws(
             x.data_ptr(), weight.data_ptr(), bias.data_ptr(), out.data_ptr(), sumsq.data_ptr(),
-            B * L, Nn, C, C, C, Nn, int(sq_cols), _stream(x.device)))
+            B * L, Nn, C, C, C, Nn, int(sq_cols), None if ws is None else ws.data_ptr(), n, _stream(x.device)))
     return out, sumsq
 
 
