@@ -61,3 +61,14 @@ def test_split(W, M, N_, K, scratch):
     squares = got[:, :C].reshape(M, C // 64, 64).square().sum(-1).t()
     # 64 positive fp32 terms
     assert ((sums[:C // 64 * M].view(C // 64, M) - squares).abs() <= squares * 65 * 2 ** -24).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [80, 2160, 2816])
+def test_ffn_down_route(W, tokens):
+    """The FFN-down projection by either GEMM: bf16 roundings of the same sums."""
+    lin = torch.nn.Linear(14336, 3072, device=DEV, dtype=torch.bfloat16).requires_grad_(False)
+    x = torch.randn(2, tokens // 2, 14336, device=DEV, generator=torch.Generator(device=DEV).manual_seed(tokens)).bfloat16()
+    got, want = W.fast_dit._linear_split_k(x, lin).double(), x.double() @ lin.weight.double().t() + lin.bias.double()
+    room = want.abs() * 2 ** -8 + (x.double().abs() @ lin.weight.double().abs().t() + 1) * 14337 * 2 ** -24
+    assert got.shape == want.shape and ((got - want).abs() <= room).all()

@@ -131,7 +131,22 @@ def _ffn_gelu_epilogue(h, ffn):
     """FFN with the tanh-GELU applied in the first GEMM's epilogue (hipBLASLt)."""
     B, L, C = h.shape
     up = torch._addmm_activation(ffn[0].bias, h.reshape(B * L, C), ffn[0].weight.t(), use_gelu=True)
-    return _linear(up.view(B, L, -1), ffn[2])
+    return _linear_split_k(up.view(B, L, -1), ffn[2])
+
+
+def _linear_split_k(x, layer):
+    """F.linear, by this library's GEMM where the product is long and its output small: up to
+    half of the CUs with one 256 x 256 tile each, which hipBLASLt runs on as many CUs as it has
+    tiles while this one splits them over k.  FFN-down (14336 -> 3072), us hipBLASLt / here:
+    80 tokens 44 / 36, 368 77 / 48, 752 107 / 82, 1080 125 / 108, 1480 146 / 131, 2160 266 / 173,
+    2360 186 / 188; beyond, 2600 193 / 201 and 4800 290 / 364."""
+    w, b = layer.weight, layer.bias
+    n, k = w.shape
+    tiles = (x.shape[0] * x.shape[1] + 255) // 256 * (n // 256)
+    if k < 8192 or not 0 < tiles <= 128 or n % 256 or k % 64 or b is None or \
+            any(t.dtype != torch.bfloat16 or not t.is_contiguous() or t.data_ptr() % 16 for t in (x, w, b)):
+        return _linear(x, layer)
+    return ops.qkv_proj_sumsq(x, w, b, 0)[0]
 
 
 # ─── attention backends: q [B, Lq, n, d], k/v [B, Lk, n, d] -> [B, Lq, n, d] ───────
