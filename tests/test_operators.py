@@ -1,0 +1,131 @@
+"""The torch operators' native kernels (csrc/torch_ops.cpp) against the Python functions that define
+the operators: the same bits for ordinary calls, and everything else as the functions have it
+(errors, empty tensors, autograd, tracing, vmap).  A call whose first tensor requires a gradient
+runs the Python function."""
+import pytest
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+B, L, H, D = 2, 37, 24, 128
+C = H * D
+
+
+def _calls(W, device, make):
+    """name -> arguments, every operator with and without its optional tensors; make(shape, dtype)."""
+    bf, f32 = torch.bfloat16, torch.float32
+    qkv = make((B, L, 3 * C), bf)
+    q, k, v = (t.unflatten(-1, (H, D)) for t in qkv.split(C, -1))
+    kc, vc = make((B, 50, H, D), bf), make((B, 50, H, D), bf)
+    long_ = [make((1, n, 2, D), bf) for n in (257, 1500, 1500)]       # a size with scratch
+    g, cos, sin = make((C,), bf), make((L, 64), f32), make((L, 64), f32)
+    lens = torch.tensor([50, 7], dtype=torch.int32, device=device)
+    inv, sums = make((B, L), f32).abs(), make((4 * H, B * L), f32).abs() * 64
+    x, y, e, e2 = make((B, L, C), bf), make((B, L, C), bf), make((1, 6, C), bf), make((1, 2, C), bf)
+    w, b = make((512, 1024), bf), make((512,), bf)
+    o = W.ops
+    return {
+        "flash_self_attn": (o.flash_self_attn, (q, k, v, 0.09, 0)),
+        "flash_self_attn_part": (o.flash_self_attn, (*long_, 0.09, 1200)),
+        "cross_attn": (o.cross_attn, (q, kc, vc, None, 0.09)),
+        "cross_attn_lens": (o.cross_attn, (q, kc, vc, lens, 0.09)),
+        "self_attn_fused": (o.self_attn_fused, (q, k, v, g, g, 1e-6, cos, sin, 0.09)),
+        "self_attn_fused_sumsq": (o.self_attn_fused_sumsq, (q, k, v, sums, g, g, 1e-6, cos, sin, 0.09)),
+        "cross_attn_fused": (o.cross_attn_fused, (q, kc, vc, g, 1e-6, None, 0.09)),
+        "cross_attn_fused_lens": (o.cross_attn_fused, (q, kc, vc, g, 1e-6, lens, 0.09)),
+        "flash_attn_qnorm": (o.flash_attn_qnorm, (q, k, v, inv, g, None, None, None, 0.09)),
+        "flash_attn_qnorm_rope": (o.flash_attn_qnorm, (q, k, v, inv, g, cos, sin, None, 0.09)),
+        "flash_attn_qnorm_lens": (o.flash_attn_qnorm, (q, kc, vc, inv, g, None, None, lens, 0.09)),
+        "rope": (o.rope, (q, cos, sin)),
+        "rms_norm": (o.rms_norm, (k, g, 1e-6)),
+        "rms_norm_rope": (o.rms_norm, (k, g, 1e-6, cos, sin)),
+        "rms_inv": (o.rms_inv, (k, 1e-6)),
+        "adaln": (o.adaln_stage, (x, y, e, 1, 2, 0, 1, None, None, 1e-6, True)),
+        "adaln_rows": (o.adaln_stage, (x, y, e, 1, 5, 0, 1, g, g, 1e-6, True, e2)),
+        "adaln_norm": (o.adaln_stage, (x, None, None, 1, -1, -1, -1, None, None, 1e-6, True)),
+        "adaln_gate": (o.adaln_stage, (x, y, e, 1, 2, -1, -1, None, None, 1e-6, False)),
+        "qkv_proj_sumsq": (o.qkv_proj_sumsq, (make((B, L, 1024), bf), w, b, 256)),
+        "qkv_proj": (o.qkv_proj_sumsq, (make((B, L, 1024), bf), w, b, 0)),
+    }
+
+
+NAMES = list(_calls(type("W", (), {"ops": type("O", (), {"__getattr__": lambda s, n: None})()}), "cpu",
+                    lambda shape, dtype: torch.zeros(shape, dtype=dtype)))
+
+
+def _tuple(r):
+    return r if isinstance(r, tuple) else (r,)
+
+
+class _Seen(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.names.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+def test_traces_on_fake_device_tensors(W):
+    """The native autograd kernel hands fake tensors on to their mode, with and without gradients."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode():
+        for name, (op, args) in _calls(W, "cuda", lambda s, dtype: torch.empty(s, dtype=dtype, device="cuda")).items():
+            for grad in (False, True):
+                out = _tuple(op(args[0].detach().requires_grad_(grad), *args[1:]))
+                assert out[0].device.type == "cuda" and out[0].requires_grad == grad, name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", NAMES)
+def test_native_equals_python(W, name):
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    make = lambda shape, dtype: torch.randn(shape, generator=gen, device="cuda").to(dtype)     # noqa: E731
+    op, args = _calls(W, "cuda", make)[name]
+    native = _tuple(op(*args))
+    python = _tuple(op(args[0].detach().requires_grad_(), *args[1:]))
+    for a, b in zip(native, python):
+        assert not a.requires_grad and a.shape == b.shape and a.stride() == b.stride() and a.dtype == b.dtype
+        if name == "qkv_proj" and a.dtype == torch.float32:
+            continue                                            # no columns asked for: not written
+        assert torch.equal(a, b.detach())
+    needs = [t for t in python if t.requires_grad]
+    assert needs
+    with pytest.raises(RuntimeError, match="no autograd formula"):
+        needs[0].sum().backward()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side), torch.inference_mode():
+        again = _tuple(op(*args))
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(again[0], native[0])
+    with _Seen() as seen:
+        op(*args)
+    assert any(s.startswith("wan_hip.") for s in seen.names)
+
+
+@pytest.mark.gpu
+def test_other_calls_as_the_functions_have_them(W):
+    o, dev = W.ops, "cuda"
+    x = torch.randn(2, 5, 2, D, device=dev).bfloat16()
+    g = torch.ones(2 * D, device=dev, dtype=torch.bfloat16)
+    cos = torch.ones(5, 64, device=dev)
+    for bad, what in ((x.float(), "bfloat16"), (x[..., :64], "head_dim"), (x[0], "expected"), (x.cpu(), "CUDA"),
+                      (x.transpose(1, 3).contiguous().transpose(1, 3), "contiguous"),
+                      (x.flatten()[1:1 + 4 * D].view(1, 2, 2, D), "aligned")):
+        with pytest.raises(ValueError, match=what):
+            o.rms_norm(bad, g, 1e-6)
+    for args in ((x, g[1:], 1e-6), (x, g, 1e-6, cos), (x, g, 1e-6, cos, cos.double()), (x, g.cpu(), 1e-6)):
+        with pytest.raises(ValueError):
+            o.rms_norm(*args)
+    with pytest.raises(ValueError, match="actual_seqlen_k"):
+        o.flash_self_attn(x, x, x, 0.1, 6)
+    with pytest.raises(ValueError, match="differ"):
+        o.cross_attn(x, x, x[:, :3], None, 0.1)
+    with pytest.raises(ValueError, match="seqlen_k"):
+        o.cross_attn(x, x, x, torch.ones(2, device=dev), 0.1)
+    with pytest.raises(RuntimeError, match=r"wan_cross_attn failed \(code 2\).*softmax_scale"):
+        o.cross_attn(x, x, x, None, -0.1)
+    assert o.rms_norm(x[:, :0], g, 1e-6).shape == (2, 0, 2, D)
+    each = torch.vmap(lambda a: o.rms_norm(a, g, 1e-6))(torch.stack([x, 2 * x]))
+    assert torch.equal(each[0], o.rms_norm(x, g, 1e-6)) and each.shape == (2, *x.shape)

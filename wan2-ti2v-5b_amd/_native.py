@@ -1,4 +1,5 @@
-"""ctypes binding of libwan_attn.so, the C ABI declared in include/wan_attn.h.
+"""ctypes binding of libwan_attn.so, the C ABI declared in include/wan_attn.h, and the loading of
+libwan_ops.so, the torch operators' native kernels over it.
 
 torch is imported first on purpose: the library is linked against the HIP
 runtime by soname (libamdhip64.so.7), and the dynamic loader resolves that to
@@ -9,10 +10,11 @@ no fallback path.
 import ctypes
 import os
 
-import torch  # noqa: F401  (must precede the CDLL load, see above)
+import torch  # (must precede the CDLL load, see above)
 
 LIB_NAME = "libwan_attn.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
+OPS_LIB_PATH = os.path.join(os.path.dirname(LIB_PATH), "libwan_ops.so")
 
 
 class WanTensor(ctypes.Structure):
@@ -69,9 +71,10 @@ def lib() -> ctypes.CDLL:
     """The loaded library (loaded on first use). Raises if it is missing or stale."""
     global _lib
     if _lib is None:
-        if not os.path.exists(LIB_PATH):
+        missing = [p for p in (LIB_PATH, OPS_LIB_PATH) if not os.path.exists(p)]
+        if missing:
             raise RuntimeError(
-                f"{LIB_PATH} is not built; run `python __graft_entry__.py build` "
+                f"{' and '.join(missing)} not built; run `python __graft_entry__.py build` "
                 "(or wan2-ti2v-5b_amd/build.py) first")
         handle = ctypes.CDLL(LIB_PATH)
         for name, (res, args) in SIGNATURES.items():
@@ -82,6 +85,13 @@ def lib() -> ctypes.CDLL:
             raise RuntimeError(f"{LIB_PATH}: ABI version {handle.wan_attn_abi_version()} != {ABI_VERSION}")
         _lib = handle
     return _lib
+
+
+def load_operators() -> None:
+    """Registers the operators' native kernels, once ops.py has defined the operators.  Before the
+    libraries are built there is nothing to register: the first call raises in lib()."""
+    if os.path.exists(LIB_PATH) and os.path.exists(OPS_LIB_PATH):
+        torch.ops.load_library(OPS_LIB_PATH)
 
 
 def last_error() -> str:

@@ -7,6 +7,10 @@ returns a new contiguous [B, Lq, H, 128] tensor.  Outputs and workspaces come
 from torch's caching allocator; the native side allocates nothing.
 
 The fake (meta) kernels let torch.compile trace the ops without running them.
+
+Ordinary calls on CUDA (HIP) tensors run in the native kernels of csrc/torch_ops.cpp, which check
+what the functions here check.  Calls that do not pass (for which the functions here raise, or
+which are empty) and calls under autograd come here.
 """
 from typing import Optional, Tuple
 
@@ -447,3 +451,6 @@ def self_attn_fused_sumsq(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sum
 @self_attn_fused_sumsq.register_fake
 def _(q, k, v, sumsq, gamma_q, gamma_k, eps, cos, sin, softmax_scale):
     return q.new_empty(q.shape)
+
+
+N.load_operators()
