@@ -8,7 +8,8 @@
   for every tile count, each operand read sees its tile landed and published by an
   earlier barrier, no copy overwrites a buffer that a slower wave may still read, the
   output staging (which reuses K buffers 0 and 1) starts only after every K read, and
-  a planted mistake in the protocol is caught.
+  a planted mistake in the protocol is caught;
+* the same for the 4-wave kernels' two buffers each with the barrier before PV.
 
 No kernel runs here; the GPU tests check the numbers the kernel produces.
 """
@@ -136,9 +137,9 @@ def _ring4_ops(n, *, drop_epilogue_barrier=False, v_ring_of_two=False, no_wait_o
     return ops
 
 
-def _check_protocol(n, **mistakes):
+def _check_protocol(n, make=_ring4_ops, **mistakes):
     phase, pending, issues, reads, epi = 0, [], [], [], None
-    for op in _ring4_ops(n, **mistakes):
+    for op in make(n, **mistakes):
         if op[0] == "bar":
             phase += 1
         elif op[0] == "issue":
@@ -163,7 +164,7 @@ def _check_protocol(n, **mistakes):
     for buf, tile, ph in reads:
         if buf[0] == "k" and buf[1] in (0, 1):
             assert ph < epi, "the output staging may overwrite a K tile still being read"
-    return sum(1 for op in _ring4_ops(n, **mistakes) if op[0] == "bar")
+    return sum(1 for op in make(n, **mistakes) if op[0] == "bar")
 
 
 @pytest.mark.parametrize("n", list(range(1, 40)) + [123])
@@ -197,3 +198,42 @@ def test_wave_without_rows_keeps_the_protocol(n):
             ops += [("wait",), ("bar",)]
     ops.append(("bar",))
     assert ops == [op for op in _ring4_ops(n) if op[0] in ("issue", "wait", "bar")]
+
+
+# ---------------------------------------------------------------------------
+# the two-buffer protocol (4 waves; the persistent kernel's items too)
+# ---------------------------------------------------------------------------
+
+def _ring2_ops(n, *, rope=False, barrier_at_end=False, no_first_barrier=False, no_last_wait=False):
+    """The per-wave sequence of the 4-wave kernels for n tiles: the barrier between the softmax
+    of a tile and its PV, the copies after it."""
+    K, V = lambda t: ("k", t % 2), lambda t: ("v", t % 2)
+    k01 = [("issue", K(t), ("K", t)) for t in (0, 1) if t < n]
+    v0 = [("issue", V(0), ("V", 0))]
+    ops = k01[:1] + v0 + k01[1:] + [("wait",), ("bar",)] if rope else k01 + [("wait",), ("bar",)] + v0
+    ops.append(("read", K(0), ("K", 0)))                 # S(0)
+    if not no_first_barrier:
+        ops.append(("bar",))
+    if n > 2:
+        ops.append(("issue", K(2), ("K", 2)))
+    for t in range(n - 1):
+        ops.append(("read", K(t + 1), ("K", t + 1)))     # S(t+1) and the softmax of tile t
+        sync = [("wait",), ("bar",)]
+        copies = ([("issue", K(t + 3), ("K", t + 3))] if t + 3 < n else []) + [("issue", V(t + 1), ("V", t + 1))]
+        pv = [("read", V(t), ("V", t))]
+        ops += copies + pv + sync if barrier_at_end else sync + copies + pv
+    ops += ([] if no_last_wait else [("wait",), ("bar",)]) + [("read", V(n - 1), ("V", n - 1)), ("epilogue",)]
+    return ops
+
+
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("n", range(1, 20))
+def test_ring2_protocol(n, rope):
+    assert _check_protocol(n, _ring2_ops, rope=rope) == 3 + (n - 1)
+
+
+@pytest.mark.parametrize("mistake", ["barrier_at_end", "no_first_barrier", "no_last_wait"])
+def test_ring2_planted_mistakes_are_caught(mistake):
+    with pytest.raises(AssertionError):
+        for n in range(1, 20):
+            _check_protocol(n, _ring2_ops, **{mistake: True})
