@@ -64,11 +64,20 @@ def test_split(W, M, N_, K, scratch):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tokens", [80, 2160, 2816])
-def test_ffn_down_route(W, tokens):
-    """The FFN-down projection by either GEMM: bf16 roundings of the same sums."""
-    lin = torch.nn.Linear(14336, 3072, device=DEV, dtype=torch.bfloat16).requires_grad_(False)
-    x = torch.randn(2, tokens // 2, 14336, device=DEV, generator=torch.Generator(device=DEV).manual_seed(tokens)).bfloat16()
-    got, want = W.fast_dit._linear_split_k(x, lin).double(), x.double() @ lin.weight.double().t() + lin.bias.double()
-    room = want.abs() * 2 ** -8 + (x.double().abs() @ lin.weight.double().abs().t() + 1) * 14337 * 2 ** -24
+@pytest.mark.parametrize("k,n,tokens", [(14336, 3072, 80), (14336, 3072, 2160), (14336, 3072, 2600), (14336, 3072, 2848),
+                                        (3072, 3072, 5504), (3072, 3072, 5502)])
+def test_projection_route(W, k, n, tokens):
+    """A projection by either GEMM: bf16 roundings of the same sums."""
+    lin = torch.nn.Linear(k, n, device=DEV, dtype=torch.bfloat16).requires_grad_(False)
+    x = torch.randn(2, tokens // 2, k, device=DEV, generator=torch.Generator(device=DEV).manual_seed(tokens)).bfloat16()
+    got, want = W.fast_dit._linear_own(x, lin).double(), x.double() @ lin.weight.double().t() + lin.bias.double()
+    room = want.abs() * 2 ** -8 + (x.double().abs() @ lin.weight.double().abs().t() + 1) * (k + 1) * 2 ** -24
     assert got.shape == want.shape and ((got - want).abs() <= room).all()
+
+
+def test_projection_route_without_library_conditions(W):
+    """Rows outside the ranges, other widths, a missing bias or another type stay torch's."""
+    for lin, rows in ((torch.nn.Linear(3072, 3072, dtype=torch.bfloat16), 4), (torch.nn.Linear(64, 32), 8),
+                      (torch.nn.Linear(14336, 3072, bias=False), 2), (torch.nn.Linear(14336, 3072), 2)):
+        x = torch.randn(1, rows, lin.in_features, dtype=lin.weight.dtype)
+        assert torch.equal(W.fast_dit._linear_own(x, lin), torch.nn.functional.linear(x, lin.weight, lin.bias))

@@ -131,19 +131,31 @@ def _ffn_gelu_epilogue(h, ffn):
     """FFN with the tanh-GELU applied in the first GEMM's epilogue (hipBLASLt)."""
     B, L, C = h.shape
     up = torch._addmm_activation(ffn[0].bias, h.reshape(B * L, C), ffn[0].weight.t(), use_gelu=True)
-    return _linear_split_k(up.view(B, L, -1), ffn[2])
+    return _linear_own(up.view(B, L, -1), ffn[2])
 
 
-def _linear_split_k(x, layer):
-    """F.linear, by this library's GEMM where the product is long and its output small: up to
-    half of the CUs with one 256 x 256 tile each, which hipBLASLt runs on as many CUs as it has
-    tiles while this one splits them over k.  FFN-down (14336 -> 3072), us hipBLASLt / here:
-    80 tokens 44 / 36, 368 77 / 48, 752 107 / 82, 1080 125 / 108, 1480 146 / 131, 2160 266 / 173,
-    2360 186 / 188; beyond, 2600 193 / 201 and 4800 290 / 364."""
+# Rows (tokens of all samples) at which the projection from k to n channels is taken to this
+# library's GEMM (ops.qkv_proj_sumsq without sums).  hipBLASLt's choice of kernel changes from size
+# to size, and where it takes one that neither splits nor streams k it runs the long FFN-down
+# product on as many CUs as it has tiles, or leaves most of the last round idle; this GEMM splits
+# those tiles.  Measured every 64 to 128 rows from 64 to 16384 with the weights from memory; inside
+# these ranges it is 5% to 45% faster, outside hipBLASLt is faster or within 5%.  us there / here:
+#   14336 -> 3072   368 77 / 48    1080 125 / 108   2160 266 / 173   4488 476 / 370   5984 753 / 417
+#                   7480 848 / 521   8976 853 / 630   9724 947 / 690   12716 1018 / 900
+#                   outside: 2600 193 / 197   3740 252 / 310   8228 591 / 576   15708 930 / 1150
+#   3072 -> 3072    5624 111 / 95   6246 113 / 97    outside: 2160 47 / 45   15708 207 / 248
+_OWN_GEMM_ROWS = {
+    (14336, 3072): ((1, 1856), (2112, 2304), (2720, 2848), (3376, 3456), (4224, 4608), (5504, 6272), (6784, 7680),
+                    (8576, 10240), (11008, 11648), (12416, 14336)),
+    (3072, 3072): ((5504, 6656),),
+}
+
+
+def _linear_own(x, layer):
+    """F.linear(x [B, L, k], ...) by the faster of the two GEMMs (bf16, no gradients)."""
     w, b = layer.weight, layer.bias
-    n, k = w.shape
-    tiles = (x.shape[0] * x.shape[1] + 255) // 256 * (n // 256)
-    if k < 8192 or not 0 < tiles <= 128 or n % 256 or k % 64 or b is None or \
+    rows = x.shape[0] * x.shape[1]
+    if not any(lo <= rows <= hi for lo, hi in _OWN_GEMM_ROWS.get((w.shape[1], w.shape[0]), ())) or b is None or \
             any(t.dtype != torch.bfloat16 or not t.is_contiguous() or t.data_ptr() % 16 for t in (x, w, b)):
         return _linear(x, layer)
     return ops.qkv_proj_sumsq(x, w, b, 0)[0]
@@ -222,14 +234,15 @@ class _FastBlock:
         B, L, C = x.shape
         fused = self.pointwise_impl == "hip" and x.is_cuda
         stage = _hip_stage if fused else _eager_stage
+        linear = _linear_own if fused else _linear
         e = self.rows(e0)
         if fused:
             x = x.contiguous()
         if h is None:
             _, h = stage(x, None, e, nf, shift=0, scale=1, ln=blk.norm1)
-        y = _linear(self._self_attention(h, cos, sin).reshape(B, L, C), blk.self_attn.o)
+        y = linear(self._self_attention(h, cos, sin).reshape(B, L, C), blk.self_attn.o)
         x, h = stage(x, y, e, nf, gate=2, ln=blk.norm3)
-        y = _linear(self._cross_attention(h, ck, cv, seqlen_k).reshape(B, L, C), blk.cross_attn.o)
+        y = linear(self._cross_attention(h, ck, cv, seqlen_k, linear).reshape(B, L, C), blk.cross_attn.o)
         x, h = stage(x, y, e, nf, shift=3, scale=4, ln=blk.norm2)
         y = (_ffn_gelu_epilogue if fused else _ffn_eager)(h, blk.ffn)
         if next_stage is None:
@@ -256,11 +269,11 @@ class _FastBlock:
         k = _rms_normalize(_linear(h, sa.k), sa.norm_k.weight, sa.norm_k.eps).view(heads)
         return _sdpa(_rope(q, cos, sin), _rope(k, cos, sin), _linear(h, sa.v).view(heads))
 
-    def _cross_attention(self, h, ck, cv, seqlen_k):
+    def _cross_attention(self, h, ck, cv, seqlen_k, linear=_linear):
         ca = self.block.cross_attn
         B, L, C = h.shape
         heads = (B, L, ca.num_heads, ca.head_dim)
-        q = _linear(h, ca.q)
+        q = linear(h, ca.q)
         if self.cross_impl == "hip":
             return ops.cross_attn_fused(q.view(heads), ck, cv, ca.norm_q.weight, ca.norm_q.eps,
                                         seqlen_k, ca.head_dim ** -0.5)
