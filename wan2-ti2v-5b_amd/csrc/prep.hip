@@ -15,6 +15,9 @@ namespace {
 
 constexpr int kMaxChunksPerLane = 16;  // supports H*128 <= 8192 channels per token
 
+// A task that only turns given partial sums into inverse RMS.
+__host__ __device__ inline bool sums_only(const PrepArgs& a) { return a.sumsq != nullptr && a.out == nullptr; }
+
 // Rotate interleaved pairs of 8 consecutive channels of one token by their four angles.
 __device__ __forceinline__ void rope8(float u[8], const f32x4 c, const f32x4 s) {
 #pragma clang fp contract(off)
@@ -78,9 +81,8 @@ __device__ __forceinline__ void rms_prep_rows(const PrepArgs& a, int block) {
     }
   }
   if (a.sumsq != nullptr) {
-    const int lane = threadIdx.x & 63;   // one partial sum a lane, in every wave of the row
-    if (lane < a.sumsq_parts) ss = a.sumsq[(int64_t)(a.sumsq_first + lane) * (a.B * a.L) + tok];
-    ss = wave_sum(ss);
+    // one partial sum a lane (64 at most) of the row's first wave
+    if (t < a.sumsq_parts) ss = a.sumsq[(int64_t)(a.sumsq_first + t) * (a.B * a.L) + tok];
   } else {
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
@@ -92,8 +94,8 @@ __device__ __forceinline__ void rms_prep_rows(const PrepArgs& a, int block) {
         }
       }
     }
-    ss = row_sum<W>(ss, 0);
   }
+  ss = row_sum<W>(ss, 0);
   const float inv = 1.0f / sqrtf(ss / (float)(a.H * kHeadDim) + a.eps);
   if (a.inv_rms != nullptr && t == 0) a.inv_rms[tok] = inv;
   if (!want) return;
@@ -120,6 +122,20 @@ __device__ __forceinline__ void rms_prep_rows(const PrepArgs& a, int block) {
   }
 }
 
+// The statistics alone, from the projection GEMM's partial sums: a thread per token, so that the
+// 64 tokens of a wave read whole lines (us with their k pass, a block per token / so: 2160 tokens
+// 8.0 / 7.0, 8228 28.0 / 22.8, 15708 52.3 / 37.7; with a loop of single loads 9.2 / 28.2 / 38.9).
+template <int W>
+__device__ __forceinline__ void inv_rms_of_sums(const PrepArgs& a, int block) {
+  const int tok = block * (64 * W) + threadIdx.x;
+  if (tok >= a.B * a.L) return;
+  const float* p = a.sumsq + (int64_t)a.sumsq_first * (a.B * a.L) + tok;
+  float ss = 0.f;
+#pragma unroll 16
+  for (int i = 0; i < a.sumsq_parts; ++i) ss += p[(int64_t)i * (a.B * a.L)];
+  a.inv_rms[tok] = 1.0f / sqrtf(ss / (float)(a.H * kHeadDim) + a.eps);
+}
+
 template <int NCH, int W, bool NT>
 __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void rms_prep_kernel(const PrepArgs a) {
   rms_prep_rows<NCH, W, NT>(a, blockIdx.x);
@@ -130,8 +146,12 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void rms_prep_kernel(const P
 template <int NCH, int W, bool NT>
 __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void rms_prep2_kernel(const PrepArgs a0, const PrepArgs a1,
                                                                          int blocks0) {
-  if ((int)blockIdx.x < blocks0) rms_prep_rows<NCH, W, NT>(a0, blockIdx.x);
-  else rms_prep_rows<NCH, W, NT>(a1, blockIdx.x - blocks0);
+  if ((int)blockIdx.x < blocks0) {
+    if (sums_only(a0)) inv_rms_of_sums<W>(a0, blockIdx.x);
+    else rms_prep_rows<NCH, W, NT>(a0, blockIdx.x);
+  } else {
+    rms_prep_rows<NCH, W, NT>(a1, blockIdx.x - blocks0);
+  }
 }
 
 // One thread per 8 channels: out = rope(x), the _rope semantics on its own.
@@ -168,7 +188,8 @@ template <int NCH, int W, bool NT>
 int launch_prep(const PrepArgs& a0, const PrepArgs* a1, hipStream_t s) {
   constexpr int R = W == 1 ? 4 : 1;   // rows per block
   const dim3 block(W == 1 ? 256 : 64 * W);
-  const int blocks0 = (a0.B * a0.L + R - 1) / R;
+  const int per0 = a1 != nullptr && sums_only(a0) ? 64 * W : R;
+  const int blocks0 = (a0.B * a0.L + per0 - 1) / per0;
   if (a1 == nullptr)
     hipLaunchKernelGGL((rms_prep_kernel<NCH, W, NT>), dim3(blocks0), block, 0, s, a0);
   else
