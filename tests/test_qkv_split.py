@@ -65,7 +65,8 @@ def test_split(W, M, N_, K, scratch):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("k,n,tokens", [(14336, 3072, 80), (14336, 3072, 2160), (14336, 3072, 2600), (14336, 3072, 2848),
-                                        (3072, 3072, 5504), (3072, 3072, 5502)])
+                                        (3072, 3072, 5504), (3072, 3072, 5502),
+                                        (3072, 18432, 12), (3072, 18432, 42)])
 def test_projection_route(W, k, n, tokens):
     """A projection by either GEMM: bf16 roundings of the same sums."""
     lin = torch.nn.Linear(k, n, device=DEV, dtype=torch.bfloat16).requires_grad_(False)

@@ -11,7 +11,7 @@ chosen once at import, under the reference's selector names (models/fast_dit.py:
                        Q-RMSNorm + masked cross-attention kernel (ops.cross_attn_fused)
   FAST_POINTWISE_IMPL  "hip" (default): each pointwise stage of a block is one fused pass
                        (ops.adaln) and GELU is the FFN-up GEMM's epilogue; "eager": torch ops
-  FAST_QKV_IMPL        with "hip" attention, the q/k/v projection: "hipblaslt" (default) or
+  FAST_QKV_IMPL        with "hip" attention, the q/k/v projection: "auto" (default), "hipblaslt" or
                        "hip", the gfx950 GEMM that also emits the QK-RMSNorm sums of squares
 
 A block (models/fast_dit.py:270-311) is organised here as four pointwise stages between
@@ -43,19 +43,19 @@ from .model import WanModel, sinusoidal_embedding_1d
 FAST_ATTN_IMPL = os.environ.get("FAST_ATTN_IMPL", "hip")
 FAST_CROSS_IMPL = os.environ.get("FAST_CROSS_IMPL", FAST_ATTN_IMPL)
 FAST_POINTWISE_IMPL = os.environ.get("FAST_POINTWISE_IMPL", "hip")
-# The fused q/k/v projection of the "hip" self-attention: "hipblaslt" (default), or "hip", the
-# gfx950 GEMM whose epilogue emits the QK-RMSNorm sums of squares (ops.qkv_proj_sumsq), so the
-# q statistics pass disappears; it measures 0.70 ms against hipBLASLt's 0.60 ms at the
-# B=2, L=7854 shape, more than the 9-20 us the q read costs, hence not the default.
-FAST_QKV_IMPL = os.environ.get("FAST_QKV_IMPL", "hipblaslt")
+# The fused q/k/v projection of the "hip" self-attention: "hipblaslt", or "hip", the gfx950 GEMM
+# whose epilogue emits the QK-RMSNorm sums of squares (ops.qkv_proj_sumsq), so the q statistics
+# pass disappears, or "auto" (default), "hip" at the token counts where that GEMM is the faster
+# one (_OWN_GEMM_ROWS; at the B=2, L=7854 shape it takes 0.69 ms against hipBLASLt's 0.61).
+FAST_QKV_IMPL = os.environ.get("FAST_QKV_IMPL", "auto")
 IMPLS = ("hip", "sdpa")
 for _name, _val in (("FAST_ATTN_IMPL", FAST_ATTN_IMPL), ("FAST_CROSS_IMPL", FAST_CROSS_IMPL)):
     if _val not in IMPLS:
         raise ValueError(f"{_name}={_val!r}: expected one of {IMPLS}")
 if FAST_POINTWISE_IMPL not in ("hip", "eager"):
     raise ValueError(f"FAST_POINTWISE_IMPL={FAST_POINTWISE_IMPL!r}: expected 'hip' or 'eager'")
-if FAST_QKV_IMPL not in ("hipblaslt", "hip"):
-    raise ValueError(f"FAST_QKV_IMPL={FAST_QKV_IMPL!r}: expected 'hipblaslt' or 'hip'")
+if FAST_QKV_IMPL not in ("auto", "hipblaslt", "hip"):
+    raise ValueError(f"FAST_QKV_IMPL={FAST_QKV_IMPL!r}: expected 'auto', 'hipblaslt' or 'hip'")
 
 
 def _linear(x, layer):
@@ -144,19 +144,29 @@ def _ffn_gelu_epilogue(h, ffn):
 #                   7480 848 / 521   8976 853 / 630   9724 947 / 690   12716 1018 / 900
 #                   outside: 2600 193 / 197   3740 252 / 310   8228 591 / 576   15708 930 / 1150
 #   3072 -> 3072    5624 111 / 95   6246 113 / 97    outside: 2160 47 / 45   15708 207 / 248
+#   3072 -> 9216    1900 118 / 97   2160 110 / 102   5624 312 / 270   8228 445 / 375   11069 516 / 477
+#                   outside: 1720 80 / 90   4192 202 / 202   6820 290 / 324   15708 613 / 690
+#   3072 -> 18432   6 64 / 31       outside: 21 26 / 31
 _OWN_GEMM_ROWS = {
     (14336, 3072): ((1, 1856), (2112, 2304), (2720, 2848), (3376, 3456), (4224, 4608), (5504, 6272), (6784, 7680),
                     (8576, 10240), (11008, 11648), (12416, 14336)),
     (3072, 3072): ((5504, 6656),),
+    (3072, 9216): ((1824, 2240), (5472, 5888), (7552, 8704), (10880, 12288)),   # q, k and v
+    (3072, 18432): ((1, 16),),                                                  # the time projection
 }
 
 
+def _own_gemm(rows, w):
+    return any(lo <= rows <= hi for lo, hi in _OWN_GEMM_ROWS.get((w.shape[1], w.shape[0]), ()))
+
+
 def _linear_own(x, layer):
-    """F.linear(x [B, L, k], ...) by the faster of the two GEMMs (bf16, no gradients)."""
+    """F.linear(x [B, L, k], ...) by the faster of the two GEMMs, for contiguous bf16 tensors on the
+    GPU that need no gradient."""
     w, b = layer.weight, layer.bias
-    rows = x.shape[0] * x.shape[1]
-    if not any(lo <= rows <= hi for lo, hi in _OWN_GEMM_ROWS.get((w.shape[1], w.shape[0]), ())) or b is None or \
-            any(t.dtype != torch.bfloat16 or not t.is_contiguous() or t.data_ptr() % 16 for t in (x, w, b)):
+    if not _own_gemm(x.shape[0] * x.shape[1], w) or b is None or not x.is_cuda or \
+            any(t.dtype != torch.bfloat16 or not t.is_contiguous() or t.data_ptr() % 16 or
+                (t.requires_grad and torch.is_grad_enabled()) for t in (x, w, b)):
         return _linear(x, layer)
     return ops.qkv_proj_sumsq(x, w, b, 0)[0]
 
@@ -221,7 +231,7 @@ class _FastBlock:
         blk = self.block
         return (blk.modulation.unsqueeze(0) + e0).reshape(self.num_frames, 6, blk.modulation.shape[-1])
 
-    def __call__(self, x, e0, cos, sin, ck, cv, seqlen_k=None, h=None, next_stage=None):
+    def __call__(self, x, e0, cos, sin, ck, cv, seqlen_k=None, h=None, next_stage=None, rows=None):
         """x [B, L, C] bf16; e0 [1, F, 6, C] time projection; cos/sin [L, 64]; ck/cv the
         block's text keys/values [B, Lc, n, d]; seqlen_k: per-sample text lengths or None.
 
@@ -229,13 +239,13 @@ class _FastBlock:
         that ended the previous block already made it; next_stage = (rows, LayerNorm, shift,
         scale) of the stage that follows this block (the next block's norm1 + modulation, or
         the output head's), done in the same pass as this block's gated residual.  Then the
-        call returns (x, h_next); otherwise x."""
+        call returns (x, h_next); otherwise x.  rows: this block's rows(e0), when at hand."""
         blk, nf = self.block, self.num_frames
         B, L, C = x.shape
         fused = self.pointwise_impl == "hip" and x.is_cuda
         stage = _hip_stage if fused else _eager_stage
         linear = _linear_own if fused else _linear
-        e = self.rows(e0)
+        e = self.rows(e0) if rows is None else rows
         if fused:
             x = x.contiguous()
         if h is None:
@@ -251,13 +261,18 @@ class _FastBlock:
         mod, ln, shift, scale = next_stage
         return stage(x, y, e, nf, gate=5, shift=shift, scale=scale, ln=ln, mod=mod)
 
+    def _own_qkv(self, h):
+        sa = self.block.self_attn
+        grad = torch.is_grad_enabled() and (h.requires_grad or sa.q.weight.requires_grad)
+        return h.dtype == torch.bfloat16 and _own_gemm(h.shape[0] * h.shape[1], self.w_qkv) and not grad
+
     def _self_attention(self, h, cos, sin):
         sa = self.block.self_attn
         B, L, C = h.shape
         heads = (B, L, sa.num_heads, sa.head_dim)
         scale = sa.head_dim ** -0.5
         if self.attn_impl == "hip":
-            if self.qkv_impl == "hip":
+            if self.qkv_impl == "hip" or (self.qkv_impl == "auto" and self._own_qkv(h)):
                 qkv, sumsq = ops.qkv_proj_sumsq(h.contiguous(), self.w_qkv, self.b_qkv, 2 * C)
                 q, k, v = (t.view(heads) for t in qkv.split(C, dim=-1))
                 return ops.self_attn_fused_sumsq(q, k, v, sumsq, sa.norm_q.weight, sa.norm_k.weight,
@@ -379,7 +394,8 @@ class FastWanDiT:
         else:
             sincos = sincos.to(self.device)
         emb = m.time_embedding(sincos.unsqueeze(0))
-        return emb, m.time_projection(emb).view(1, self.num_frames, 6, m.dim)
+        silu, project = m.time_projection
+        return emb, _linear_own(silu(emb), project).view(1, self.num_frames, 6, m.dim)
 
     def patch(self, latent):
         """Patch embedding (a Conv3d with stride = kernel = patch_size) as one GEMM: gather
@@ -404,14 +420,15 @@ class FastWanDiT:
         x = self.patch(latent)
         m = self.model
         n = len(self.blocks)
-        h = None
+        h, rows = None, None
         for i, (blk, (ck, cv)) in enumerate(zip(self.blocks, self.context)):
             if i + 1 < n:
                 nxt = self.blocks[i + 1]
                 following = (nxt.rows(e0), nxt.block.norm1, 0, 1)
             else:
                 following = (head_rows(m.head, e, self.num_frames), m.head.norm, 0, 1)
-            x, h = blk(x, e0, self.cos, self.sin, ck, cv, self.seqlen_k, h=h, next_stage=following)
+            x, h = blk(x, e0, self.cos, self.sin, ck, cv, self.seqlen_k, h=h, next_stage=following, rows=rows)
+            rows = following[0]
         return noise_prediction(m.head, x, e, self.grid, m.patch_size, m.out_dim, self.guide_scale, h=h)
 
 
