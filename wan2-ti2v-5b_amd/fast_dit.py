@@ -139,18 +139,19 @@ def _ffn_gelu_epilogue(h, ffn):
 # to size, and where it takes one that neither splits nor streams k it runs the long FFN-down
 # product on as many CUs as it has tiles, or leaves most of the last round idle; this GEMM splits
 # those tiles.  Measured every 64 to 128 rows from 64 to 16384 with the weights from memory; inside
-# these ranges it is 5% to 45% faster, outside hipBLASLt is faster or within 5%.  us there / here:
+# these ranges it is 4% to 45% faster, outside hipBLASLt is faster or within 5%.  us there / here:
 #   14336 -> 3072   368 77 / 48    1080 125 / 108   2160 266 / 173   4488 476 / 370   5984 753 / 417
 #                   7480 848 / 521   8976 853 / 630   9724 947 / 690   12716 1018 / 900
 #                   outside: 2600 193 / 197   3740 252 / 310   8228 591 / 576   15708 930 / 1150
-#   3072 -> 3072    5624 111 / 95   6246 113 / 97    outside: 2160 47 / 45   15708 207 / 248
+#   3072 -> 3072    2160 47 / 45   2440 51 / 46   5624 111 / 95   6246 113 / 97   outside: 2600 51 / 49
+#                   15708 207 / 248
 #   3072 -> 9216    1900 118 / 97   2160 110 / 102   5624 312 / 270   8228 445 / 375   11069 516 / 477
 #                   outside: 1720 80 / 90   4192 202 / 202   6820 290 / 324   15708 613 / 690
 #   3072 -> 18432   6 64 / 31       outside: 21 26 / 31
 _OWN_GEMM_ROWS = {
     (14336, 3072): ((1, 1856), (2112, 2304), (2720, 2848), (3376, 3456), (4224, 4608), (5504, 6272), (6784, 7680),
                     (8576, 10240), (11008, 11648), (12416, 14336)),
-    (3072, 3072): ((5504, 6656),),
+    (3072, 3072): ((2112, 2480), (5504, 6656)),
     (3072, 9216): ((1824, 2240), (5472, 5888), (7552, 8704), (10880, 12288)),   # q, k and v
     (3072, 18432): ((1, 16),),                                                  # the time projection
 }
