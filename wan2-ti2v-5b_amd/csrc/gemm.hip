@@ -371,10 +371,15 @@ __global__ __launch_bounds__(256) void gemm_merge_kernel(const GemmArgs a, int r
   });
 }
 
-// Tile heights: the x rows of a workgroup's tile, and what a round of such tiles (one workgroup
-// per CU) takes, in us: per 64 of k, and besides (weights from memory, fitted over M 80 to 15708).
-constexpr struct { int rows; float k_us; } kTiles[] = {{320, 1.78f}, {256, 1.58f}, {192, 1.27f}, {128, 0.79f}};
-constexpr float kRoundUs = 10.f;
+// Tile heights: the x rows of a workgroup's tile, and what a full round of such tiles (one
+// workgroup per CU) takes, in us: per 64 of k, and besides (fitted over M 40 to 15708).
+constexpr struct { int rows; float k_us; bool power; } kTiles[] = {
+    {320, 1.86f, true}, {256, 1.55f, true}, {192, 1.32f, true}, {128, 0.81f, false}};
+constexpr float kRoundUs = 6.f;
+// A round that fills only a share of the CUs runs at a higher clock (256 rows, N 9216: a second
+// round of 0.11, 0.27, 0.55, 0.69 and 0.97 of the CUs takes 54, 58, 62, 67 and 83 us, a full one
+// 78); tiles of 128 rows wait for their copies and gain nothing.
+float round_share(float fill, bool power) { return power ? 0.66f + 0.25f * fill + 0.1f * fill * fill : 1.f; }
 // The merge launch, and the write and read of a part's row of 256 fp32 (plain stores: past the
 // L2s, non-temporally, the calls took 3-7 us longer).
 constexpr float kMergeUs = 4.f, kMergeRowUs = 2 * 256 * 4 / 8e6f;
@@ -387,15 +392,15 @@ struct GemmPlan {
   float us;
 };
 
-// The plan whose rounds take least, with up to `scratch` bytes for the parts.  A round that is
-// mostly empty costs what a full one costs, so between two heights the number of rounds decides,
-// and where a last (or only) round leaves half of the CUs or more idle, its tiles may be split
-// over k: the parts' fp32 sums cost a merge launch and their way through memory.  us, tiles of
-// 256 rows alone / the best height / as chosen here:
-//   N 9216, K 3072:   M 80  59 / 45 / 28   M 256  58 / 48 / 32   M 2160  137 / 104 / 104 (320 rows)
-//                     M 8228  376 / 374 / 374 (320)   M 15708  756 / 756 / 690 (320, a tail of 8 tiles)
-//   N 3072, K 14336:  M 80  - / 182 / 36   M 748  - / 178 / 82   M 1500  - / 173 / 132
-//                     M 2160  - / 187 / 173 (320 rows, three parts)   M 8228  - / 739 / 581
+// The plan whose rounds take least, with up to `scratch` bytes for the parts.  Between two heights
+// the number of rounds decides, and where a last (or only) round leaves half of the CUs or more
+// idle, its tiles may be split over k: the parts' fp32 sums cost a merge launch and their way
+// through memory.  us, tiles of 256 rows alone / as chosen here:
+//   N 9216, K 3072:   M 80  56 / 23   M 256  58 / 28   M 896  60 / 46   M 2170  136 / 98 (320 rows)
+//                     M 2280  136 / 124 (a tail of 68 tiles, three parts)   M 2940  145 (256 rows)
+//                     M 4480  222 / 194 (320)   M 8228  370 / 358 (320)   M 15708  702 / 684
+//   N 3072, K 14336 (the best height unsplit / as chosen):   M 80  182 / 36   M 748  178 / 82
+//                     M 1500  173 / 132   M 2160  187 / 172 (320 rows, three parts)   M 8228  739 / 581
 GemmPlan gemm_plan(int M, int N, int K, int cus, size_t scratch) {
   GemmPlan best{0, 0, 0, 1, 0.f};
   const int kt = K / kGemmBK;
@@ -406,7 +411,7 @@ GemmPlan gemm_plan(int M, int N, int K, int cus, size_t scratch) {
     for (int n = 1; n == 1 || (rest > 0 && n <= kMaxSplits && rest * n <= cus && n * kMinSplitTiles <= kt); ++n) {
       if (n > 1 && (size_t)rest * n * t.rows * GBN * sizeof(float) > scratch) break;
       float us = full * (kt * t.k_us + kRoundUs);
-      if (rest > 0) us += (kt + n - 1) / n * t.k_us + kRoundUs;
+      if (rest > 0) us += ((kt + n - 1) / n * t.k_us + kRoundUs) * round_share((float)(rest * n) / cus, t.power);
       if (n > 1) us += kMergeUs + (float)rest * n * t.rows * kMergeRowUs;
       if (best.rows == 0 || us < best.us) best = {t.rows, n > 1 ? (int)(tiles - rest) : 0, n > 1 ? rest : 0, n, us};
     }
