@@ -259,10 +259,12 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmA
   // splits around the barrier that publishes the next tile: NM - NF MFMAs, the wait for
   // that tile's copies (those of later tiles stay in flight) and the barrier, then NF
   // MFMAs, each followed by a read of the next tile's first k-step.
-  int slot = 0;                       // of tile kt
+  int ring = 0;                       // slot of tile kt, with more than two
   auto tile = [&](int kt, auto next_c, auto copy_c) {
     constexpr bool has_next = decltype(next_c)::value, has_copy = decltype(copy_c)::value;
-    const int nslot = slot == SLOTS - 1 ? 0 : slot + 1, cslot = slot == 0 ? SLOTS - 1 : slot - 1;
+    const int slot = SLOTS == 2 ? kt & 1 : ring;
+    const int nslot = SLOTS == 2 ? slot ^ 1 : slot == SLOTS - 1 ? 0 : slot + 1;
+    const int cslot = SLOTS == 2 ? slot ^ 1 : slot == 0 ? SLOTS - 1 : slot - 1;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const int cur = ks & 1, nxt = cur ^ 1;
@@ -291,7 +293,7 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_rowsq_kernel(const GemmA
         for (int i = NM; i < NC; ++i) copy_one(cslot, kt + SLOTS - 1, i);
       }
     }
-    slot = nslot;
+    ring = nslot;
   };
 
   for (int t = 0; t < SLOTS - 1 && t < kt_count; ++t)
