@@ -1,6 +1,6 @@
 """GPU: wan_qkv_proj_sumsq at the edges of its tile heights (128, 192, 256 and 320 rows of x),
-against float64.  With N = 9216 (36 column tiles) and 256 CUs the launcher takes 128 rows up to
-M 896, 192 up to 1344, 256 up to 1792 and 320 up to 2240."""
+against float64.  With N = 9216 (36 column tiles), K = 1024 and 256 CUs the launcher takes 128 rows
+from M 193, 192 from 897, 256 from 1345 and 320 from 1793; shorter products choose differently."""
 import pytest
 import torch
 
@@ -9,10 +9,10 @@ DEV = torch.device("cuda:0")
 
 
 @pytest.mark.parametrize("M,K", [
-    (1, 64), (127, 128), (128, 192), (129, 256), (896, 64),      # 128 rows: 1 to 4 tiles of k in 3 slots
-    (897, 64), (1152, 128), (1153, 192),                         # 192
-    (1345, 64), (1536, 128), (1537, 320),                        # 256
-    (1793, 64), (1920, 128), (1921, 192), (2240, 3072),          # 320
+    (769, 192), (896, 192), (577, 256), (193, 1024), (896, 1024),       # 128 rows: 3, 4 and 16 tiles of k in 3 slots
+    (1, 64), (192, 128), (897, 1024), (1153, 1024), (1344, 1024),       # 192
+    (193, 64), (1345, 1024), (1537, 1024), (1792, 1024),                # 256
+    (577, 64), (1537, 128), (1793, 1024), (1921, 1024), (2240, 3072),   # 320
 ])
 def test_tile_heights(W, M, K):
     N_, C = 9216, 6144
