@@ -1,0 +1,36 @@
+"""The launch plans of csrc/plans.h (host arithmetic) as ctypes functions: compiled with the host
+compiler behind a few C entry points, for the tests of launchers without a device."""
+import ctypes
+import os
+import subprocess
+import tempfile
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "wan2-ti2v-5b_amd", "csrc")
+SHIM = """
+#include "plans.h"
+using namespace wan;
+extern "C" {
+void gemm(int M, int N, int K, long long ldx, int cus, size_t scratch, int* out, size_t* bytes) {
+  const GemmPlan p = gemm_plan(M, N, K, ldx, cus, scratch);
+  out[0] = p.rows; out[1] = p.from; out[2] = p.rest; out[3] = p.splits;
+  *bytes = gemm_plan_bytes(p);
+}
+}
+"""
+
+
+def load() -> ctypes.CDLL:
+    with tempfile.TemporaryDirectory() as d:
+        src, lib = os.path.join(d, "plans.cpp"), os.path.join(d, "plans.so")
+        with open(src, "w") as f:
+            f.write(SHIM)
+        subprocess.run([os.environ.get("CXX", "g++"), "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC",
+                        "-I", CSRC, src, "-o", lib], check=True)
+        return ctypes.CDLL(lib)
+
+
+def gemm(lib, M, N, K, ldx=None, cus=256, scratch=0):
+    """(tile rows, whole tiles before the split, split tiles, parts of each, scratch bytes)"""
+    out, n = (ctypes.c_int * 4)(), ctypes.c_size_t()
+    lib.gemm(M, N, K, ctypes.c_longlong(K if ldx is None else ldx), cus, ctypes.c_size_t(scratch), out, ctypes.byref(n))
+    return (*out, n.value)

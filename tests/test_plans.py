@@ -1,0 +1,35 @@
+"""The launch plans (csrc/plans.h) over sizes that no device is needed for."""
+import plans
+import pytest
+
+
+@pytest.fixture(scope="module")
+def lib():
+    return plans.load()
+
+
+# wan_qkv_proj_sumsq accepts row strides of x below 2^23 elements; a tile's rows are copied from 32-bit
+# byte offsets (row * stride * 2, and up to 128 bytes of k).  320 rows: 319 * 2 * 6731904 + 128 = 2^32 - 5120
+@pytest.mark.parametrize("ldx,tall", [(3072, True), (6731904, True), (6731912, False), (7000000, False),
+                                      ((1 << 23) - 8, False)])
+def test_gemm_tiles_end_within_their_offsets(lib, ldx, tall):
+    assert (plans.gemm(lib, 2160, 9216, 3072, ldx)[0] == 320) == tall
+
+
+@pytest.mark.parametrize("ldx", [6731904, 6731912, 7500000, (1 << 23) - 8])
+def test_gemm_offsets_fit_at_every_size(lib, ldx):
+    for scratch in (0, 1 << 30):
+        for M in [1, 2, 255, 256, 257, 319, 320, 321] + list(range(400, 16000, 117)):
+            for N, K in ((9216, 3072), (3072, 14336), (3072, 3072), (512, 64)):
+                rows = plans.gemm(lib, M, N, K, ldx, scratch=scratch)[0]
+                assert rows in (128, 192, 256, 320)
+                assert (min(rows, M) - 1) * ldx * 2 + 128 <= 1 << 32, (M, N, K, rows)
+
+
+def test_gemm_plan_is_the_same_with_ordinary_strides(lib, W):
+    """... and its scratch is what wan_qkv_proj_workspace asks for (256 CUs without a device)."""
+    ws = W._native.lib().wan_qkv_proj_workspace
+    for M in range(1, 9000, 61):
+        for N, K in ((9216, 3072), (3072, 14336), (3072, 3072)):
+            p = plans.gemm(lib, M, N, K, scratch=1 << 40)
+            assert p == plans.gemm(lib, M, N, K, 3 * K, scratch=1 << 40) and p[4] == ws(M, N, K)

@@ -529,7 +529,8 @@ int wan_qkv_proj_sumsq_ws(const void* x, const void* w, const void* bias, void* 
   if (ldx < K || ldw < K || ldo < N || ldx % 8 || ldw % 8 || ldo % 8)
     return set_error(WAN_ERR_INVALID, "%s: row strides (%lld, %lld, %lld) must cover the rows and be "
                      "multiples of 8 elements", fn, (long long)ldx, (long long)ldw, (long long)ldo);
-  // a tile's 256 rows are addressed with 32-bit byte offsets
+  // a tile's rows are addressed with 32-bit byte offsets: 256 rows with any stride below this, and
+  // the launcher takes no taller tile than the stride leaves room for
   if (ldx >= (int64_t(1) << 23) || ldw >= (int64_t(1) << 23))
     return set_error(WAN_ERR_UNSUPPORTED, "%s: row strides must be below 2^23 elements", fn);
   // x, w, bias and out are always read or written when M > 0; sumsq only when sq_cols > 0

@@ -35,6 +35,7 @@
 // traffic, one wave per SIMD) run the loop at a higher clock (1.72 vs 1.58 GHz) but in
 // more cycles per tile, and tie with this tiling at best.
 #include "launchers.h"
+#include "plans.h"
 
 #include <type_traits>
 
@@ -42,11 +43,11 @@ namespace wan {
 
 namespace {
 
-constexpr int GBN = 256;
+constexpr int GBN = kGemmCols;
 constexpr int kGroupM = 8;
 // 8 waves in a 2 x 4 grid (each 128 x 64 of a 256 x 256 tile, two waves per SIMD),
 // 64 k per stage: measured the fastest of 2 x 2 / 2 x 4 waves, 32 / 64 k, 2-5 stages
-constexpr int kGemmWM = 2, kGemmWN = 4, kGemmBK = 64;
+constexpr int kGemmWM = 2, kGemmWN = 4;
 
 __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
@@ -373,56 +374,6 @@ __global__ __launch_bounds__(256) void gemm_merge_kernel(const GemmArgs a, int r
   });
 }
 
-// Tile heights: the x rows of a workgroup's tile, and what a full round of such tiles (one
-// workgroup per CU) takes, in us: per 64 of k, and besides (fitted over M 40 to 15708).
-constexpr struct { int rows; float k_us; bool power; } kTiles[] = {
-    {320, 1.86f, true}, {256, 1.55f, true}, {192, 1.32f, true}, {128, 0.81f, false}};
-constexpr float kRoundUs = 6.f;
-// A round that fills only a share of the CUs runs at a higher clock (256 rows, N 9216: a second
-// round of 0.11, 0.27, 0.55, 0.69 and 0.97 of the CUs takes 54, 58, 62, 67 and 83 us, a full one
-// 78); tiles of 128 rows wait for their copies and gain nothing.
-float round_share(float fill, bool power) { return power ? 0.66f + 0.25f * fill + 0.1f * fill * fill : 1.f; }
-// The merge launch, and the write and read of a part's row of 256 fp32 (plain stores: past the
-// L2s, non-temporally, the calls took 3-7 us longer).
-constexpr float kMergeUs = 4.f, kMergeRowUs = 2 * 256 * 4 / 8e6f;
-constexpr int kMaxSplits = 16, kMinSplitTiles = 4;
-
-// How a product is run: tiles of `rows` rows, the first `from` of them whole, the `rest` as
-// `splits` parts over k each.
-struct GemmPlan {
-  int rows, from, rest, splits;
-  float us;
-};
-
-// The plan whose rounds take least, with up to `scratch` bytes for the parts.  Between two heights
-// the number of rounds decides, and where a last (or only) round leaves half of the CUs or more
-// idle, its tiles may be split over k: the parts' fp32 sums cost a merge launch and their way
-// through memory.  us, tiles of 256 rows alone / as chosen here:
-//   N 9216, K 3072:   M 80  56 / 23   M 256  58 / 28   M 896  60 / 46   M 2170  136 / 98 (320 rows)
-//                     M 2280  136 / 124 (a tail of 68 tiles, three parts)   M 2940  145 (256 rows)
-//                     M 4480  222 / 194 (320)   M 8228  370 / 358 (320)   M 15708  702 / 684
-//   N 3072, K 14336 (the best height unsplit / as chosen):   M 80  182 / 36   M 748  178 / 82
-//                     M 1500  173 / 132   M 2160  187 / 172 (320 rows, three parts)   M 8228  739 / 581
-GemmPlan gemm_plan(int M, int N, int K, int cus, size_t scratch) {
-  GemmPlan best{0, 0, 0, 1, 0.f};
-  const int kt = K / kGemmBK;
-  for (const auto& t : kTiles) {
-    const int64_t tiles = ((int64_t)M + t.rows - 1) / t.rows * (N / GBN);
-    const int64_t full = tiles / cus;
-    const int rest = (int)(tiles % cus);
-    for (int n = 1; n == 1 || (rest > 0 && n <= kMaxSplits && rest * n <= cus && n * kMinSplitTiles <= kt); ++n) {
-      if (n > 1 && (size_t)rest * n * t.rows * GBN * sizeof(float) > scratch) break;
-      float us = full * (kt * t.k_us + kRoundUs);
-      if (rest > 0) us += ((kt + n - 1) / n * t.k_us + kRoundUs) * round_share((float)(rest * n) / cus, t.power);
-      if (n > 1) us += kMergeUs + (float)rest * n * t.rows * kMergeRowUs;
-      if (best.rows == 0 || us < best.us) best = {t.rows, n > 1 ? (int)(tiles - rest) : 0, n > 1 ? rest : 0, n, us};
-    }
-  }
-  return best;
-}
-
-size_t plan_bytes(const GemmPlan& p) { return p.splits > 1 ? (size_t)p.rest * p.splits * p.rows * GBN * sizeof(float) : 0; }
-
 template <int GBM, int SLOTS>
 int launch_rows(const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
   const int64_t tiles = ((int64_t)a.M + GBM - 1) / GBM * (a.N / GBN);
@@ -447,12 +398,12 @@ int launch_rows(const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
 
 size_t gemm_split_bytes(int M, int N, int K) {
   if (M <= 0 || N < GBN || K < kGemmBK) return 0;
-  return plan_bytes(gemm_plan(M, N, K, device_cu_count(), SIZE_MAX));
+  return gemm_plan_bytes(gemm_plan(M, N, K, K, device_cu_count(), SIZE_MAX));
 }
 
 int launch_gemm_rowsq(const GemmArgs& a, hipStream_t s) {
   if (a.M == 0) return 0;
-  GemmPlan p = gemm_plan(a.M, a.N, a.K, device_cu_count(), a.part != nullptr ? a.part_bytes : 0);
+  const GemmPlan p = gemm_plan(a.M, a.N, a.K, a.ldx, device_cu_count(), a.part != nullptr ? a.part_bytes : 0);
   // as many slots as the 160 KB of LDS hold
   switch (p.rows) {
     case 320: return launch_rows<320, 2>(a, p, s);

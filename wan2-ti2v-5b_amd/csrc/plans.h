@@ -1,0 +1,77 @@
+// How launches are laid out: sizes in, tiles, parts and grids out.  Host arithmetic only, so that
+// it can be checked over any sizes without a device.
+#pragma once
+
+#include <cstddef>
+#include <cstdint>
+
+namespace wan {
+
+// ---------------------------------------------------------------------------
+// the projection GEMM (gemm.hip)
+// ---------------------------------------------------------------------------
+
+// Columns of an output tile and k per stage.
+constexpr int kGemmCols = 256, kGemmBK = 64;
+
+// Tile heights: the x rows of a workgroup's tile, and what a full round of such tiles (one
+// workgroup per CU) takes, in us: per 64 of k, and besides (fitted over M 40 to 15708).
+constexpr struct { int rows; float k_us; bool power; } kTiles[] = {
+    {320, 1.86f, true}, {256, 1.55f, true}, {192, 1.32f, true}, {128, 0.81f, false}};
+constexpr float kRoundUs = 6.f;
+// A round that fills only a share of the CUs runs at a higher clock (256 rows, N 9216: a second
+// round of 0.11, 0.27, 0.55, 0.69 and 0.97 of the CUs takes 54, 58, 62, 67 and 83 us, a full one
+// 78); tiles of 128 rows wait for their copies and gain nothing.
+inline float round_share(float fill, bool power) { return power ? 0.66f + 0.25f * fill + 0.1f * fill * fill : 1.f; }
+// The merge launch, and the write and read of a part's row of 256 fp32 (plain stores: past the
+// L2s, non-temporally, the calls took 3-7 us longer).
+constexpr float kMergeUs = 4.f, kMergeRowUs = 2 * 256 * 4 / 8e6f;
+constexpr int kGemmMaxSplits = 16, kMinSplitTiles = 4;
+
+// The rows of a tile of x are copied from 32-bit byte offsets of its first: whether the last row's
+// last byte has one.  wan_qkv_proj_sumsq takes row strides below 2^23 elements, with which it has
+// in tiles of up to 256 rows; 320 rows end at 6731904 elements.
+inline bool tile_addressable(int M, int rows, int64_t ldx) {
+  return (int64_t)((M < rows ? M : rows) - 1) * ldx * 2 + kGemmBK * 2 <= int64_t(1) << 32;
+}
+
+// How a product is run: tiles of `rows` rows, the first `from` of them whole, the `rest` as
+// `splits` parts over k each.
+struct GemmPlan {
+  int rows, from, rest, splits;
+  float us;
+};
+
+// The plan whose rounds take least, with up to `scratch` bytes for the parts, for x rows `ldx`
+// elements apart.  Between two heights the number of rounds decides, and where a last (or only)
+// round leaves half of the CUs or more idle, its tiles may be split over k: the parts' fp32 sums
+// cost a merge launch and their way through memory.  us, tiles of 256 rows alone / as chosen here:
+//   N 9216, K 3072:   M 80  56 / 23   M 256  58 / 28   M 896  60 / 46   M 2170  136 / 98 (320 rows)
+//                     M 2280  136 / 124 (a tail of 68 tiles, three parts)   M 2940  145 (256 rows)
+//                     M 4480  222 / 194 (320)   M 8228  370 / 358 (320)   M 15708  702 / 684
+//   N 3072, K 14336 (the best height unsplit / as chosen):   M 80  182 / 36   M 748  178 / 82
+//                     M 1500  173 / 132   M 2160  187 / 172 (320 rows, three parts)   M 8228  739 / 581
+inline GemmPlan gemm_plan(int M, int N, int K, int64_t ldx, int cus, size_t scratch) {
+  GemmPlan best{0, 0, 0, 1, 0.f};
+  const int kt = K / kGemmBK;
+  for (const auto& t : kTiles) {
+    if (!tile_addressable(M, t.rows, ldx)) continue;
+    const int64_t tiles = ((int64_t)M + t.rows - 1) / t.rows * (N / kGemmCols);
+    const int64_t full = tiles / cus;
+    const int rest = (int)(tiles % cus);
+    for (int n = 1; n == 1 || (rest > 0 && n <= kGemmMaxSplits && rest * n <= cus && n * kMinSplitTiles <= kt); ++n) {
+      if (n > 1 && (size_t)rest * n * t.rows * kGemmCols * sizeof(float) > scratch) break;
+      float us = full * (kt * t.k_us + kRoundUs);
+      if (rest > 0) us += ((kt + n - 1) / n * t.k_us + kRoundUs) * round_share((float)(rest * n) / cus, t.power);
+      if (n > 1) us += kMergeUs + (float)rest * n * t.rows * kMergeRowUs;
+      if (best.rows == 0 || us < best.us) best = {t.rows, n > 1 ? (int)(tiles - rest) : 0, n > 1 ? rest : 0, n, us};
+    }
+  }
+  return best;
+}
+
+inline size_t gemm_plan_bytes(const GemmPlan& p) {
+  return p.splits > 1 ? (size_t)p.rest * p.splits * p.rows * kGemmCols * sizeof(float) : 0;
+}
+
+}  // namespace wan
