@@ -9,14 +9,14 @@ def lib():
 
 
 # wan_qkv_proj_sumsq accepts row strides of x below 2^23 elements; a tile's rows are copied from 32-bit
-# byte offsets (row * stride * 2, and up to 128 bytes of k).  320 rows: 319 * 2 * 6731904 + 128 = 2^32 - 5120
-@pytest.mark.parametrize("ldx,tall", [(3072, True), (6731904, True), (6731912, False), (7000000, False),
+# byte offsets (row * stride * 2, and up to 128 bytes of k).  320 rows: 319 * 2 * 6731920 + 128 = 2^32 - 2208
+@pytest.mark.parametrize("ldx,tall", [(3072, True), (6731920, True), (6731928, False), (7000000, False),
                                       ((1 << 23) - 8, False)])
 def test_gemm_tiles_end_within_their_offsets(lib, ldx, tall):
     assert (plans.gemm(lib, 2160, 9216, 3072, ldx)[0] == 320) == tall
 
 
-@pytest.mark.parametrize("ldx", [6731904, 6731912, 7500000, (1 << 23) - 8])
+@pytest.mark.parametrize("ldx", [6731920, 6731928, 7500000, (1 << 23) - 8])
 def test_gemm_offsets_fit_at_every_size(lib, ldx):
     for scratch in (0, 1 << 30):
         for M in [1, 2, 255, 256, 257, 319, 320, 321] + list(range(400, 16000, 117)):

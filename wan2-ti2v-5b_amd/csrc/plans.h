@@ -30,7 +30,7 @@ constexpr int kGemmMaxSplits = 16, kMinSplitTiles = 4;
 
 // The rows of a tile of x are copied from 32-bit byte offsets of its first: whether the last row's
 // last byte has one.  wan_qkv_proj_sumsq takes row strides below 2^23 elements, with which it has
-// in tiles of up to 256 rows; 320 rows end at 6731904 elements.
+// in tiles of up to 256 rows; 320 rows end at 6731920 elements.
 inline bool tile_addressable(int M, int rows, int64_t ldx) {
   return (int64_t)((M < rows ? M : rows) - 1) * ldx * 2 + kGemmBK * 2 <= int64_t(1) << 32;
 }
