@@ -45,6 +45,7 @@ def _calls(W, device, make):
         "adaln_gate": (o.adaln_stage, (x, y, e, 1, 2, -1, -1, None, None, 1e-6, False)),
         "qkv_proj_sumsq": (o.qkv_proj_sumsq, (make((B, L, 1024), bf), w, b, 256)),
         "qkv_proj": (o.qkv_proj_sumsq, (make((B, L, 1024), bf), w, b, 0)),
+        "linear": (o.linear, (make((B, L, 1024), bf), w, b)),
     }
 
 
@@ -129,3 +130,31 @@ def test_other_calls_as_the_functions_have_them(W):
     assert o.rms_norm(x[:, :0], g, 1e-6).shape == (2, 0, 2, D)
     each = torch.vmap(lambda a: o.rms_norm(a, g, 1e-6))(torch.stack([x, 2 * x]))
     assert torch.equal(each[0], o.rms_norm(x, g, 1e-6)) and each.shape == (2, *x.shape)
+
+
+def test_linear_is_torchs_where_the_kernel_does_not_take_it(W):
+    """Other devices, types, layouts and sizes: torch's bits."""
+    F = torch.nn.functional
+    for x, w, b in ((torch.randn(2, 3, 64), torch.randn(256, 64), torch.randn(256)),
+                    (torch.randn(2, 3, 65).bfloat16(), torch.randn(7, 65).bfloat16(), torch.randn(7).bfloat16()),
+                    (torch.randn(5, 64).bfloat16(), torch.randn(256, 64).bfloat16(), torch.randn(256).bfloat16()),
+                    (torch.randn(2, 0, 64), torch.randn(256, 64), torch.randn(256))):
+        assert torch.equal(W.ops.linear(x, w, b), F.linear(x, w, b))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("which", ["weight", "bias", "x"])
+def test_linear_misaligned_is_torchs(W, which):
+    """2560 and 2561 values from the start of an allocation: the address decides, and every operand that
+    F.linear takes is taken."""
+    t = {n: torch.randn(*s, device="cuda").bfloat16() for n, s in (("x", (2, 5, 64)), ("weight", (256, 64)), ("bias", (256,)))}
+    flat = torch.zeros(t[which].numel() + 2561, device="cuda", dtype=torch.bfloat16)
+    for off in (2560, 2561):
+        view = flat[off:off + t[which].numel()].view(t[which].shape)
+        view.copy_(t[which])
+        args = {**t, which: view}
+        got, want = W.ops.linear(**args).double(), args["x"].double() @ args["weight"].double().t() + args["bias"].double()
+        assert ((got - want).abs() <= want.abs() * 2 ** -8 + 1e-3).all()
+        if off % 8:
+            assert torch.equal(W.ops.linear(**args), torch.nn.functional.linear(**{"input": args["x"], "weight": args["weight"],
+                                                                                     "bias": args["bias"]}))

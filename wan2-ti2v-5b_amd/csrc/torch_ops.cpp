@@ -358,13 +358,34 @@ void qkv_proj_sumsq(const OperatorHandle& op, DispatchKeySet ks, Stack* stack) {
   c.give(std::move(out), std::move(sumsq));
 }
 
+// linear(x, weight, bias): what the kernel does not take (a misaligned weight among it) is torch's, in
+// the Python function
+void linear(const OperatorHandle& op, DispatchKeySet ks, Stack* stack) {
+  Call c(op, stack);
+  const Tensor &x = c.tensor(0), &w = c.tensor(1), &b = c.tensor(2);
+  const auto dev = x.device();
+  if (!dev.is_cuda() || x.dim() != 3 || w.dim() != 2 || !block(x, x.sizes(), dev) ||
+      !block(w, {w.size(0), x.size(2)}, dev) || !block(b, {w.size(0)}, dev) || w.size(0) % 256 != 0 ||
+      x.size(2) % 64 != 0 || x.size(2) >= int64_t(1) << 23 || !small_int(x.size(0) * x.size(1)) ||
+      !small_int(w.size(0)))
+    return to_python(op, ks, stack);
+  const int M = (int)(x.size(0) * x.size(1)), N = (int)w.size(0), K = (int)x.size(2);
+  const Site s(x);
+  Tensor out = at::empty({x.size(0), x.size(1), N}, s.bf16);
+  const Scratch ws(s, wan_qkv_proj_workspace(M, N, K));
+  check("wan_qkv_proj_sumsq",
+        wan_qkv_proj_sumsq_ws(x.data_ptr(), w.data_ptr(), b.data_ptr(), out.data_ptr(), nullptr, M, N, K, K, K, N, 0,
+                              ws.ptr(), ws.n, s.stream()));
+  c.give(std::move(out));
+}
+
 }  // namespace
 
 #define WAN_OPS(X)                                                                                  \
   X("flash_self_attn", flash_self_attn) X("cross_attn", cross_attn) X("self_attn_fused", self_attn_fused) \
   X("self_attn_fused_sumsq", self_attn_fused_sumsq) X("cross_attn_fused", cross_attn_fused)         \
   X("flash_attn_qnorm", flash_attn_qnorm) X("rope", rope_op) X("rms_norm", rms_norm) X("rms_inv", rms_inv) \
-  X("adaln", adaln) X("qkv_proj_sumsq", qkv_proj_sumsq)
+  X("adaln", adaln) X("qkv_proj_sumsq", qkv_proj_sumsq) X("linear", linear)
 
 TORCH_LIBRARY_IMPL(wan_hip, CUDA, m) {
 #define WAN_IMPL(name, fn) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&fn>());

@@ -135,7 +135,7 @@ def _ffn_gelu_epilogue(h, ffn):
 
 
 # Rows (tokens of all samples) at which the projection from k to n channels is taken to this
-# library's GEMM (ops.qkv_proj_sumsq without sums).  hipBLASLt's choice of kernel changes from size
+# library's GEMM (ops.linear).  hipBLASLt's choice of kernel changes from size
 # to size, and where it takes one that neither splits nor streams k it runs the long FFN-down
 # product on as many CUs as it has tiles, or leaves most of the last round idle; this GEMM splits
 # those tiles.  Measured every 64 to 128 rows from 64 to 16384 with the weights from memory; inside
@@ -158,18 +158,22 @@ _OWN_GEMM_ROWS = {
 
 
 def _own_gemm(rows, w):
+    """Whether a projection by w of this many rows is this library's.  Traced, it is hipBLASLt's: the
+    traced graph may be run with other row counts, and F.linear in it is open to the compiler."""
+    if torch.compiler.is_compiling():
+        return False
     return any(lo <= rows <= hi for lo, hi in _OWN_GEMM_ROWS.get((w.shape[1], w.shape[0]), ()))
 
 
 def _linear_own(x, layer):
     """F.linear(x [B, L, k], ...) by the faster of the two GEMMs, for contiguous bf16 tensors on the
-    GPU that need no gradient."""
+    GPU that need no gradient (ops.linear looks at the alignment)."""
     w, b = layer.weight, layer.bias
     if not _own_gemm(x.shape[0] * x.shape[1], w) or b is None or not x.is_cuda or \
-            any(t.dtype != torch.bfloat16 or not t.is_contiguous() or t.data_ptr() % 16 or
-                (t.requires_grad and torch.is_grad_enabled()) for t in (x, w, b)):
+            any(t.dtype != torch.bfloat16 or not t.is_contiguous() or (t.requires_grad and torch.is_grad_enabled())
+                for t in (x, w, b)):
         return _linear(x, layer)
-    return ops.qkv_proj_sumsq(x, w, b, 0)[0]
+    return ops.linear(x, w, b)
 
 
 # ─── attention backends: q [B, Lq, n, d], k/v [B, Lk, n, d] -> [B, Lq, n, d] ───────
@@ -265,7 +269,9 @@ class _FastBlock:
     def _own_qkv(self, h):
         sa = self.block.self_attn
         grad = torch.is_grad_enabled() and (h.requires_grad or sa.q.weight.requires_grad)
-        return h.dtype == torch.bfloat16 and _own_gemm(h.shape[0] * h.shape[1], self.w_qkv) and not grad
+        # (storage_offset: an h handed in from elsewhere may start anywhere; F.linear takes that too)
+        return h.dtype == torch.bfloat16 and _own_gemm(h.shape[0] * h.shape[1], self.w_qkv) and not grad and \
+            h.storage_offset() % 8 == 0
 
     def _self_attention(self, h, cos, sin):
         sa = self.block.self_attn

@@ -415,6 +415,34 @@ def _(x, weight, bias, sq_cols):
             x.new_empty((max(sq_cols // 64, 1), B * L), dtype=torch.float32))
 
 
+@torch.library.custom_op("wan_hip::linear", mutates_args=())
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
+    """F.linear(x [B, L, C], weight [N, C], bias [N]), by the GEMM of qkv_proj_sumsq for the operands
+    which that takes, and by torch for all others (another alignment of a weight among them, which
+    only the running kernel can see: under tracing there are no addresses)."""
+    M, C, Nn = x.shape[:-1].numel(), x.shape[-1], weight.shape[0]
+    ts = (x, weight, bias)
+    if x.dim() != 3 or weight.shape != (Nn, C) or bias.shape != (Nn,) or M == 0 or Nn % 256 or C % 64 or Nn * C == 0 or \
+            max(M, Nn) >= 2 ** 31 or C >= 2 ** 23 or x.device.type != "cuda" or \
+            any(t.dtype != torch.bfloat16 or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16
+                for t in ts):
+        return torch.nn.functional.linear(x, weight, bias)
+    out = torch.empty((*x.shape[:2], Nn), dtype=x.dtype, device=x.device)
+    lib = N.lib()
+    with torch.cuda.device(x.device):
+        n = lib.wan_qkv_proj_workspace(M, Nn, C)
+        ws = torch.empty(n, dtype=torch.uint8, device=x.device) if n else None
+        N.check("wan_qkv_proj_sumsq", lib.wan_qkv_proj_sumsq_ws(
+            x.data_ptr(), weight.data_ptr(), bias.data_ptr(), out.data_ptr(), None, M, Nn, C, C, C, Nn, 0,
+            None if ws is None else ws.data_ptr(), n, _stream(x.device)))
+    return out
+
+
+@linear.register_fake
+def _(x, weight, bias):
+    return x.new_empty((*x.shape[:-1], weight.shape[0]))
+
+
 @torch.library.custom_op("wan_hip::self_attn_fused_sumsq", mutates_args=())
 def self_attn_fused_sumsq(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sumsq: torch.Tensor,
                           gamma_q: torch.Tensor, gamma_k: torch.Tensor, eps: float,
