@@ -281,3 +281,20 @@ def test_chained_block_boundaries_equal_separate_stages(W):
         x = blk(x, e0, fast.cos, fast.sin, ck, cv, fast.seqlen_k)
     want = W.fast_dit.noise_prediction(m.head, x, e, grid, m.patch_size, m.out_dim, 5.0)
     assert torch.equal(got, want)
+
+
+def test_time_projection_is_called_as_a_module(W):
+    """Hooks on the time projection and its layers run, and a module put in its place is called."""
+    fast = W.fast_dit.FastWanDiT(_tiny(W), (2, 2, 2), 5.0, attn_impl="sdpa", cross_impl="sdpa", pointwise_impl="eager")
+    proj, ran = fast.model.time_projection, []
+    for part in (proj, *proj):
+        part.register_forward_hook(lambda mod, args, out: ran.append(type(mod).__name__))
+    _, rows = fast.time_rows(500)
+    assert ran == ["SiLU", "Linear", "Sequential"]
+
+    class Twice(torch.nn.Module):
+        def forward(self, emb):
+            return 2 * proj(emb)
+
+    fast.model.time_projection = Twice()
+    assert torch.equal(fast.time_rows(500)[1], 2 * rows)

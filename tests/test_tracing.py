@@ -5,6 +5,7 @@ import warnings
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
 
 def _block(W, tokens, frames, dtype=torch.bfloat16):
@@ -59,3 +60,40 @@ def test_block_on_fake_tensors(W, tokens, frames):
         warnings.simplefilter("error")
         fb, args = _block(W, tokens, frames)
         assert fb(*args).shape == args[0].shape
+
+
+class _Names(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.names = set()
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.names.add(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("impl,pointwise", [("sdpa", "eager"), ("hip", "hip")])
+def test_torch_side_runs_torch_alone(W, impl, pointwise, monkeypatch):
+    """With attention "sdpa" and pointwise "eager" nothing of this library runs on the device, in the
+    blocks or around them (2160 tokens, where the other side takes its own kernels throughout)."""
+    cfg, grid = W.model.WanConfig(), (6, 12, 15)
+    monkeypatch.setattr(torch.Tensor, "pin_memory", lambda t: t)      # fake tensors have no pinned form
+    monkeypatch.setattr(W.fast_dit, "_sdpa", lambda q, *rest: torch.empty_like(q))      # asks for a device
+    torch.set_default_dtype(torch.bfloat16)
+    try:
+        with FakeTensorMode(), torch.no_grad():
+            with torch.device("cuda"):
+                m = W.model.WanModel(cfg, num_layers=1)
+            fast = W.fast_dit.FastWanDiT.__new__(W.fast_dit.FastWanDiT)
+            fast.model, fast.grid, fast.num_frames, fast.device = m, grid, grid[0], torch.device("cuda")
+            fb = W.fast_dit._FastBlock(m.blocks[0], grid[0], impl, impl, pointwise)
+            _, args = _block(W, 2160, grid[0])
+            with _Names() as seen:
+                fast.time_rows(500)
+                before = {n for n in seen.names if n.startswith("wan_hip.")}
+                fb(*args)
+    finally:
+        torch.set_default_dtype(torch.float32)
+    assert not before
+    own = {n for n in seen.names if n.startswith("wan_hip.")}
+    assert bool(own) == (impl == "hip"), own

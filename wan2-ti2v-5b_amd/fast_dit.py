@@ -10,7 +10,9 @@ chosen once at import, under the reference's selector names (models/fast_dit.py:
   FAST_CROSS_IMPL      the cross-attention backend (default: FAST_ATTN_IMPL); "hip" runs the
                        Q-RMSNorm + masked cross-attention kernel (ops.cross_attn_fused)
   FAST_POINTWISE_IMPL  "hip" (default): each pointwise stage of a block is one fused pass
-                       (ops.adaln) and GELU is the FFN-up GEMM's epilogue; "eager": torch ops
+                       (ops.adaln), GELU is the FFN-up GEMM's epilogue, and the projections after
+                       them are the gfx950 GEMM at some token counts (_OWN_GEMM_ROWS); "eager":
+                       torch ops and F.linear alone
   FAST_QKV_IMPL        with "hip" attention, the q/k/v projection: "auto" (default), "hipblaslt" or
                        "hip", the gfx950 GEMM that also emits the QK-RMSNorm sums of squares
 
@@ -147,13 +149,11 @@ def _ffn_gelu_epilogue(h, ffn):
 #                   15708 207 / 248
 #   3072 -> 9216    1900 118 / 97   2160 110 / 102   5624 312 / 270   8228 445 / 375   11069 516 / 477
 #                   outside: 1720 80 / 90   4192 202 / 202   6820 290 / 324   15708 613 / 690
-#   3072 -> 18432   6 64 / 31       outside: 21 26 / 31
 _OWN_GEMM_ROWS = {
     (14336, 3072): ((1, 1856), (2112, 2304), (2720, 2848), (3376, 3456), (4224, 4608), (5504, 6272), (6784, 7680),
                     (8576, 10240), (11008, 11648), (12416, 14336)),
     (3072, 3072): ((2112, 2480), (5504, 6656)),
     (3072, 9216): ((1824, 2240), (5472, 5888), (7552, 8704), (10880, 12288)),   # q, k and v
-    (3072, 18432): ((1, 16),),                                                  # the time projection
 }
 
 
@@ -401,8 +401,7 @@ class FastWanDiT:
         else:
             sincos = sincos.to(self.device)
         emb = m.time_embedding(sincos.unsqueeze(0))
-        silu, project = m.time_projection
-        return emb, _linear_own(silu(emb), project).view(1, self.num_frames, 6, m.dim)
+        return emb, m.time_projection(emb).view(1, self.num_frames, 6, m.dim)
 
     def patch(self, latent):
         """Patch embedding (a Conv3d with stride = kernel = patch_size) as one GEMM: gather
