@@ -69,3 +69,30 @@ def test_adaln_channels(W, C, rows):
     # roundings of the norm (2^-9 and the sums' order), of its product (2^-9) and of the result
     size = (n * s1).abs()
     assert ((h.double() - (n * s1 + sh)).abs() <= size * (2 ** -7 + 2 ** -9) + (size + sh.abs()) * 2 ** -8 + 1e-6).all()
+
+
+# 2 H partial sums a token; four rows to a block up to 4 heads (8 from 1025 rows of both tasks on),
+# where a block of the q side, 256 tokens, is not its waves times 64
+@pytest.mark.parametrize("H", [1, 4, 5, 8, 9, 24, 32])
+@pytest.mark.parametrize("tokens", [1, 63, 65, 255, 257, 512, 513, 769])
+def test_statistics_from_sums(W, H, tokens):
+    """wan_rms_norm_qk_sumsq: q's inverse RMS of every token, and k normalised by its own sums."""
+    N, s = W._native, torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=DEV).manual_seed(H * tokens)
+    sums = torch.rand(4 * H, tokens, generator=g, device=DEV) * 128
+    k = _bf((1, tokens, H, D), H + tokens)
+    gamma = 1 + _bf((H * D,), 7).abs()
+    ones, zeros = torch.ones(tokens, 64, device=DEV), torch.zeros(tokens, 64, device=DEV)
+    khat = torch.full((tokens + 1, H, D), 7.0, dtype=torch.bfloat16, device=DEV)      # margins that stay as they are
+    inv = torch.full((tokens + 64,), 7.0, device=DEV)
+    N.check("sums", N.lib().wan_rms_norm_qk_sumsq(N.tensor4(k), khat.data_ptr(), 1, tokens, H, D, gamma.data_ptr(), 1e-6,
+                                                  ones.data_ptr(), zeros.data_ptr(), sums.data_ptr(), inv.data_ptr(), s))
+    want = (sums.double().unflatten(0, (2, 2 * H)).sum(1) / (H * D) + 1e-6).rsqrt()      # q's, k's
+    # 2 H positive fp32 terms in any order, the division, the square root and the reciprocal
+    assert ((inv[:tokens].double() - want[0]).abs() <= want[0] * (H + 3) * 2 ** -24).all()
+    assert (inv[tokens:] == 7).all() and (khat[tokens:] == 7).all()
+    n = (k[0].double() * want[1][:, None, None]).to(torch.bfloat16)
+    u = (n * gamma.view(H, D)).double()
+    # an ulp of the norm where the sums' order flips it, and its product's (as test_normalised_rows)
+    assert ((khat[:tokens].double() - u).abs() <= u.abs() * 2 ** -6).all()
+    assert float((khat[:tokens].double() != u).double().mean()) < 1e-2 or u.numel() < 1e4

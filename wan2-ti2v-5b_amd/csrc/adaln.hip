@@ -41,7 +41,7 @@ namespace {
 // XCD's L2 keeps them for the next kernel, and the launch does not end with their write-back
 // (2160 rows, gate + modulate 13.6 -> 12.0 us, norm 8.6 -> 7.4; 8228 rows 41 -> 35).
 template <int NCH, int W, bool STREAM>
-__global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void adaln_kernel(const AdaLNArgs a) {
+__global__ __launch_bounds__(row_threads(W)) void adaln_kernel(const AdaLNArgs a) {
   // No contraction into FMAs: each product and sum is rounded to bf16 where the
   // separate torch ops round it (the compiler otherwise fuses ln * s1 + shift
   // across the intermediate bf16 conversion).
@@ -159,9 +159,9 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void adaln_kernel(const AdaL
 template <int NCH, int W, bool STREAM>
 int launch(const AdaLNArgs& a, hipStream_t s) {
   const int64_t tokens = (int64_t)a.B * a.L;
-  const int64_t grid = W == 1 ? (tokens + 3) / 4 : tokens;
+  const int64_t grid = (tokens + rows_per_block(W) - 1) / rows_per_block(W);
   if (grid > 0x7fffffff) return set_error(2, "adaln: %lld tokens is too many", (long long)tokens);
-  hipLaunchKernelGGL((adaln_kernel<NCH, W, STREAM>), dim3((unsigned)grid), dim3(W == 1 ? 256 : 64 * W), 0, s, a);
+  hipLaunchKernelGGL((adaln_kernel<NCH, W, STREAM>), dim3((unsigned)grid), dim3(row_threads(W)), 0, s, a);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : set_error(4, "adaln launch: %s", hipGetErrorString(e));
 }

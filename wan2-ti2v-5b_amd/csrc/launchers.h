@@ -6,6 +6,10 @@
 
 namespace wan {
 
+// The row kernels' blocks: the W waves of one token row, with a wave a row (W = 1) four rows.
+constexpr int rows_per_block(int W) { return W == 1 ? 4 : 1; }
+constexpr int row_threads(int W) { return 64 * W * rows_per_block(W); }
+
 // The sum of v over the W waves that work on one token row; `slot` names a sum of its own
 // where a kernel forms several (W = 1: the wave alone, no barrier).
 template <int W>

@@ -127,7 +127,7 @@ __device__ __forceinline__ void rms_prep_rows(const PrepArgs& a, int block) {
 // 8.0 / 7.0, 8228 28.0 / 22.8, 15708 52.3 / 37.7; with a loop of single loads 9.2 / 28.2 / 38.9).
 template <int W>
 __device__ __forceinline__ void inv_rms_of_sums(const PrepArgs& a, int block) {
-  const int tok = block * (64 * W) + threadIdx.x;
+  const int tok = block * row_threads(W) + threadIdx.x;
   if (tok >= a.B * a.L) return;
   const float* p = a.sumsq + (int64_t)a.sumsq_first * (a.B * a.L) + tok;
   float ss = 0.f;
@@ -137,15 +137,15 @@ __device__ __forceinline__ void inv_rms_of_sums(const PrepArgs& a, int block) {
 }
 
 template <int NCH, int W, bool NT>
-__global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void rms_prep_kernel(const PrepArgs a) {
+__global__ __launch_bounds__(row_threads(W)) void rms_prep_kernel(const PrepArgs a) {
   rms_prep_rows<NCH, W, NT>(a, blockIdx.x);
 }
 
 // Two independent tasks (the q statistics and the k norm + rotation of one
 // self-attention call) in one launch: blocks [0, blocks0) run a0, the rest a1.
 template <int NCH, int W, bool NT>
-__global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void rms_prep2_kernel(const PrepArgs a0, const PrepArgs a1,
-                                                                         int blocks0) {
+__global__ __launch_bounds__(row_threads(W)) void rms_prep2_kernel(const PrepArgs a0, const PrepArgs a1,
+                                                                   int blocks0) {
   if ((int)blockIdx.x < blocks0) {
     if (sums_only(a0)) inv_rms_of_sums<W>(a0, blockIdx.x);
     else rms_prep_rows<NCH, W, NT>(a0, blockIdx.x);
@@ -186,9 +186,9 @@ constexpr int64_t kStreamBytes = int64_t(128) << 20;
 // Launches `a0` alone (a1 null) or both tasks.
 template <int NCH, int W, bool NT>
 int launch_prep(const PrepArgs& a0, const PrepArgs* a1, hipStream_t s) {
-  constexpr int R = W == 1 ? 4 : 1;   // rows per block
-  const dim3 block(W == 1 ? 256 : 64 * W);
-  const int per0 = a1 != nullptr && sums_only(a0) ? 64 * W : R;
+  constexpr int R = rows_per_block(W);
+  const dim3 block(row_threads(W));
+  const int per0 = a1 != nullptr && sums_only(a0) ? row_threads(W) : R;
   const int blocks0 = (a0.B * a0.L + per0 - 1) / per0;
   if (a1 == nullptr)
     hipLaunchKernelGGL((rms_prep_kernel<NCH, W, NT>), dim3(blocks0), block, 0, s, a0);
