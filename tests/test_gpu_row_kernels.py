@@ -96,3 +96,20 @@ def test_statistics_from_sums(W, H, tokens):
     # an ulp of the norm where the sums' order flips it, and its product's (as test_normalised_rows)
     assert ((khat[:tokens].double() - u).abs() <= u.abs() * 2 ** -6).all()
     assert float((khat[:tokens].double() != u).double().mean()) < 1e-2 or u.numel() < 1e4
+
+
+@pytest.mark.parametrize("H", [1, 7, 8, 24, 32])
+def test_statistics_from_sums_keep_small_terms(W, H):
+    """One partial sum of 1 before 2 H - 1 of just under half its last place: a chain of additions
+    loses every one of them, sums in a tree of 8 levels lose 8 roundings."""
+    N, s, tokens = W._native, torch.cuda.current_stream().cuda_stream, 300
+    sums = torch.full((4 * H, tokens), 2.0 ** -24 * 0.99, device=DEV)
+    sums[0] = sums[2 * H] = 1.0
+    k, gamma = _bf((1, tokens, H, D), H), torch.ones(H * D, dtype=torch.bfloat16, device=DEV)
+    ones, zeros = torch.ones(tokens, 64, device=DEV), torch.zeros(tokens, 64, device=DEV)
+    khat, inv = torch.empty_like(k), torch.empty(tokens, device=DEV)
+    N.check("sums", N.lib().wan_rms_norm_qk_sumsq(N.tensor4(k), khat.data_ptr(), 1, tokens, H, D, gamma.data_ptr(), 0.0,
+                                                  ones.data_ptr(), zeros.data_ptr(), sums.data_ptr(), inv.data_ptr(), s))
+    want = (sums[:2 * H].double().sum(0) / (H * D)).rsqrt()
+    # half of 8 roundings of the sum, the division's, the square root's and the reciprocal's
+    assert ((inv.double() - want).abs() <= want * (4 + 2.5) * 2 ** -24).all()

@@ -130,9 +130,21 @@ __device__ __forceinline__ void inv_rms_of_sums(const PrepArgs& a, int block) {
   const int tok = block * row_threads(W) + threadIdx.x;
   if (tok >= a.B * a.L) return;
   const float* p = a.sumsq + (int64_t)a.sumsq_first * (a.B * a.L) + tok;
-  float ss = 0.f;
-#pragma unroll 16
-  for (int i = 0; i < a.sumsq_parts; ++i) ss += p[(int64_t)i * (a.B * a.L)];
+  // sixteen sums side by side, then their tree: no partial sum takes part in more than 8 roundings (a
+  // wave's tree 6; one chain of 64, 63)
+  float t[16] = {};
+  int i = 0;
+  for (; i + 16 <= a.sumsq_parts; i += 16)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) t[j] += p[(int64_t)(i + j) * (a.B * a.L)];
+#pragma unroll
+  for (int j = 0; j < 16; ++j)
+    if (i + j < a.sumsq_parts) t[j] += p[(int64_t)(i + j) * (a.B * a.L)];
+#pragma unroll
+  for (int n = 8; n > 0; n /= 2)
+#pragma unroll
+    for (int j = 0; j < n; ++j) t[j] += t[j + n];
+  const float ss = t[0];
   a.inv_rms[tok] = 1.0f / sqrtf(ss / (float)(a.H * kHeadDim) + a.eps);
 }
 
