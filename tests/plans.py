@@ -10,6 +10,11 @@ SHIM = """
 #include "plans.h"
 using namespace wan;
 extern "C" {
+void rows(long long blocks, int threads, unsigned* out) {
+  const RowGrid g = row_grid(blocks, threads);
+  out[0] = g.x; out[1] = g.y;
+}
+int threads(int W) { return row_threads(W); }
 void gemm(int M, int N, int K, long long ldx, int cus, size_t scratch, int* out, size_t* bytes) {
   const GemmPlan p = gemm_plan(M, N, K, ldx, cus, scratch);
   out[0] = p.rows; out[1] = p.from; out[2] = p.rest; out[3] = p.splits;
@@ -34,3 +39,10 @@ def gemm(lib, M, N, K, ldx=None, cus=256, scratch=0):
     out, n = (ctypes.c_int * 4)(), ctypes.c_size_t()
     lib.gemm(M, N, K, ctypes.c_longlong(K if ldx is None else ldx), cus, ctypes.c_size_t(scratch), out, ctypes.byref(n))
     return (*out, n.value)
+
+
+def rows(lib, blocks, threads):
+    """(workgroups along x, along y)"""
+    out = (ctypes.c_uint * 2)()
+    lib.rows(ctypes.c_longlong(blocks), threads, out)
+    return tuple(out)

@@ -113,3 +113,15 @@ def test_statistics_from_sums_keep_small_terms(W, H):
     want = (sums[:2 * H].double().sum(0) / (H * D)).rsqrt()
     # half of 8 roundings of the sum, the division's, the square root's and the reciprocal's
     assert ((inv.double() - want).abs() <= want * (4 + 2.5) * 2 ** -24).all()
+
+
+def test_more_rows_than_a_line_of_the_grid(W):
+    """2^32 / 128 rows of 1152 channels (two waves a row) and one batch entry more, and 2^32 / 64 rows of 8
+    (one wave): the launch goes on along y."""
+    x = _bf((1, 1024, 9, D), 3)
+    inv = W.ops.rms_inv(x.expand(32769, -1, -1, -1), 1e-6)
+    assert (inv == W.ops.rms_inv(x.expand(2, -1, -1, -1), 1e-6)[0]).all()      # (2048 rows: the same form)
+    del inv
+    x = _bf((1, 1024, 8), 4)
+    _, h = W.ops.adaln(x.expand(65537, -1, -1).contiguous())
+    assert (h == W.ops.adaln(x)[1]).all()

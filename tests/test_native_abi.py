@@ -248,3 +248,14 @@ def test_qkv_gemm_and_sumsq_prep_validation_without_launching(W):
     assert prep(t, P, 1, 16, 40, 128, P, 1e-6, P, P, P, P, None) == 2 and "partial sums" in N.last_error()
     assert prep(t, P, 1, 16, 24, 64, P, 1e-6, P, P, P, P, None) == 2 and "head_dim" in N.last_error()
     assert prep(t, P, 0, 16, 24, 128, P, 1e-6, P, P, P, P, None) == 0
+
+
+def test_rows_that_do_not_fit_an_int_are_refused(W):
+    """2^31 rows and more (2^32, whose product is 0 in 32 bits, among them)."""
+    N = W._native
+    lib, t = N.lib(), N.WanTensor(256, 0, 128, 128)
+    for batch, rows in ((65536, 65536), (65536, 32768)):
+        rc = lib.wan_rms_norm(t, None, batch, rows, 1, 128, None, 1e-6, None, None, 256, None)
+        assert rc == 2 and "rows" in N.last_error()
+        rc = lib.wan_rms_norm_qk(t, t, 256, batch, rows, 1, 128, 256, 1e-6, 256, 256, 256, None)
+        assert rc == 2 and "rows" in N.last_error()

@@ -33,3 +33,17 @@ def test_gemm_plan_is_the_same_with_ordinary_strides(lib, W):
         for N, K in ((9216, 3072), (3072, 14336), (3072, 3072)):
             p = plans.gemm(lib, M, N, K, scratch=1 << 40)
             assert p == plans.gemm(lib, M, N, K, 3 * K, scratch=1 << 40) and p[4] == ws(M, N, K)
+
+
+@pytest.mark.parametrize("waves", [1, 2, 3, 4, 6, 8])
+def test_row_grid(lib, waves):
+    """Workgroups for every row, fewer than 2^32 threads along x (what a launch takes) at any row count,
+    one line where they fit, and at most a line's end too many."""
+    threads = lib.threads(waves)
+    assert threads == (256 if waves == 1 else 64 * waves)
+    line = (2 ** 32 - 1) // threads
+    for blocks in (1, 2, 15708, line - 1, line, line + 1, 22 * 10 ** 6, 33 * 10 ** 6, 3 * line + 7, 2 ** 31 - 1, 2 ** 32 - 1):
+        x, y = plans.rows(lib, blocks, threads)
+        assert x * threads < 2 ** 32 and y < 2 ** 16
+        assert blocks <= x * y < blocks + y
+        assert y == 1 or blocks > line

@@ -47,7 +47,8 @@ __global__ __launch_bounds__(row_threads(W)) void adaln_kernel(const AdaLNArgs a
   // across the intermediate bf16 conversion).
 #pragma clang fp contract(off)
   const int t = W == 1 ? threadIdx.x & 63 : threadIdx.x;
-  const int64_t tok = W == 1 ? (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6) : (int64_t)blockIdx.x;
+  const int64_t block = row_block(a.grid_x);
+  const int64_t tok = W == 1 ? block * 4 + (threadIdx.x >> 6) : block;
   if (tok >= (int64_t)a.B * a.L) return;
   const int l = (int)(tok % a.L);
   const int f = l / (a.L / a.F);
@@ -157,11 +158,12 @@ __global__ __launch_bounds__(row_threads(W)) void adaln_kernel(const AdaLNArgs a
 }
 
 template <int NCH, int W, bool STREAM>
-int launch(const AdaLNArgs& a, hipStream_t s) {
+int launch(AdaLNArgs a, hipStream_t s) {
   const int64_t tokens = (int64_t)a.B * a.L;
-  const int64_t grid = (tokens + rows_per_block(W) - 1) / rows_per_block(W);
-  if (grid > 0x7fffffff) return set_error(2, "adaln: %lld tokens is too many", (long long)tokens);
-  hipLaunchKernelGGL((adaln_kernel<NCH, W, STREAM>), dim3((unsigned)grid), dim3(row_threads(W)), 0, s, a);
+  const RowGrid grid = row_grid((tokens + rows_per_block(W) - 1) / rows_per_block(W), row_threads(W));
+  if (grid.y > 0xffff) return set_error(2, "adaln: %lld tokens is too many", (long long)tokens);
+  a.grid_x = grid.x;
+  hipLaunchKernelGGL((adaln_kernel<NCH, W, STREAM>), dim3(grid.x, grid.y), dim3(row_threads(W)), 0, s, a);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : set_error(4, "adaln launch: %s", hipGetErrorString(e));
 }

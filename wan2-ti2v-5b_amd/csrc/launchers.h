@@ -3,12 +3,13 @@
 #pragma once
 
 #include "common.h"
+#include "plans.h"
 
 namespace wan {
 
-// The row kernels' blocks: the W waves of one token row, with a wave a row (W = 1) four rows.
-constexpr int rows_per_block(int W) { return W == 1 ? 4 : 1; }
-constexpr int row_threads(int W) { return 64 * W * rows_per_block(W); }
+// The number of a row kernel's workgroup: its grid goes on along y where x ends (row_grid), `grid_x`
+// workgroups to a line.
+__device__ __forceinline__ int64_t row_block(unsigned grid_x) { return (int64_t)blockIdx.y * grid_x + blockIdx.x; }
 
 // The sum of v over the W waves that work on one token row; `slot` names a sum of its own
 // where a kernel forms several (W = 1: the wave alone, no barrier).
@@ -41,6 +42,7 @@ struct PrepArgs {
   // partials sumsq[(sumsq_first + p) * B * L + token], p < sumsq_parts (null: from x).
   const float* sumsq;
   int sumsq_first, sumsq_parts;
+  unsigned grid_x;      // workgroups along x of the launch (set by the launcher)
 };
 int launch_rms_prep(const PrepArgs& a, hipStream_t s);
 // Two tasks with the same H in one launch.
@@ -71,6 +73,7 @@ struct AdaLNArgs {
   const bf16* ln_w;     // [C] LayerNorm affine weight / bias (null: not affine)
   const bf16* ln_b;
   float eps;
+  unsigned grid_x;      // workgroups along x of the launch (set by the launcher)
 };
 int launch_adaln(const AdaLNArgs& a, hipStream_t s);
 

@@ -8,6 +8,25 @@
 namespace wan {
 
 // ---------------------------------------------------------------------------
+// the token-row kernels (prep.hip, adaln.hip)
+// ---------------------------------------------------------------------------
+
+// Their blocks: the W waves of one token row, with a wave a row (W = 1) four rows.
+constexpr int rows_per_block(int W) { return W == 1 ? 4 : 1; }
+constexpr int row_threads(int W) { return 64 * W * rows_per_block(W); }
+
+// The grid of `blocks` workgroups of `threads`.  A launch has fewer than 2^32 threads along x (22
+// million rows of 3072 channels at three waves a row): what is over goes on along y, with up to a
+// line's last workgroups too many.
+struct RowGrid {
+  uint32_t x, y;
+};
+inline RowGrid row_grid(int64_t blocks, int threads) {
+  const int64_t line = 0xffffffffll / threads, y = (blocks + line - 1) / line;
+  return {(uint32_t)((blocks + y - 1) / y), (uint32_t)y};
+}
+
+// ---------------------------------------------------------------------------
 // the projection GEMM (gemm.hip)
 // ---------------------------------------------------------------------------
 

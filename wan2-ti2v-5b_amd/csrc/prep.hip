@@ -9,6 +9,8 @@
 // rounded as the separate torch ops round it.
 #include "launchers.h"
 
+#include <algorithm>
+
 namespace wan {
 
 namespace {
@@ -47,10 +49,11 @@ __device__ __forceinline__ void rope8(float u[8], const f32x4 c, const f32x4 s) 
 // 8228 rows 22.0 -> 20.1); with more than the last-level cache takes of rows read and written
 // they cost (15708 rows 36.6 -> 38.9).
 template <int NCH, int W, bool NT>
-__device__ __forceinline__ void rms_prep_rows(const PrepArgs& a, int block) {
+__device__ __forceinline__ void rms_prep_rows(const PrepArgs& a, unsigned block) {
   const int t = W == 1 ? threadIdx.x & 63 : threadIdx.x;
-  const int tok = W == 1 ? block * 4 + (threadIdx.x >> 6) : block;
-  if (tok >= a.B * a.L) return;
+  const unsigned row_id = W == 1 ? block * 4 + (threadIdx.x >> 6) : block;
+  if (row_id >= (unsigned)(a.B * a.L)) return;
+  const int tok = (int)row_id;
   const int b = tok / a.L, l = tok - b * a.L;
   const int nchunks = a.H * 16;
   const bf16* row = a.x.ptr + b * a.x.sb + (int64_t)l * a.x.st;
@@ -126,9 +129,9 @@ __device__ __forceinline__ void rms_prep_rows(const PrepArgs& a, int block) {
 // 64 tokens of a wave read whole lines (us with their k pass, a block per token / so: 2160 tokens
 // 8.0 / 7.0, 8228 28.0 / 22.8, 15708 52.3 / 37.7; with a loop of single loads 9.2 / 28.2 / 38.9).
 template <int W>
-__device__ __forceinline__ void inv_rms_of_sums(const PrepArgs& a, int block) {
-  const int tok = block * row_threads(W) + threadIdx.x;
-  if (tok >= a.B * a.L) return;
+__device__ __forceinline__ void inv_rms_of_sums(const PrepArgs& a, unsigned block) {
+  const unsigned tok = block * row_threads(W) + threadIdx.x;
+  if (tok >= (unsigned)(a.B * a.L)) return;
   const float* p = a.sumsq + (int64_t)a.sumsq_first * (a.B * a.L) + tok;
   // sixteen sums side by side, then their tree: no partial sum takes part in more than 8 roundings (a
   // wave's tree 6; one chain of 64, 63)
@@ -150,19 +153,20 @@ __device__ __forceinline__ void inv_rms_of_sums(const PrepArgs& a, int block) {
 
 template <int NCH, int W, bool NT>
 __global__ __launch_bounds__(row_threads(W)) void rms_prep_kernel(const PrepArgs a) {
-  rms_prep_rows<NCH, W, NT>(a, blockIdx.x);
+  rms_prep_rows<NCH, W, NT>(a, (unsigned)row_block(a.grid_x));
 }
 
 // Two independent tasks (the q statistics and the k norm + rotation of one
 // self-attention call) in one launch: blocks [0, blocks0) run a0, the rest a1.
 template <int NCH, int W, bool NT>
 __global__ __launch_bounds__(row_threads(W)) void rms_prep2_kernel(const PrepArgs a0, const PrepArgs a1,
-                                                                   int blocks0) {
-  if ((int)blockIdx.x < blocks0) {
-    if (sums_only(a0)) inv_rms_of_sums<W>(a0, blockIdx.x);
-    else rms_prep_rows<NCH, W, NT>(a0, blockIdx.x);
+                                                                   unsigned blocks0) {
+  const unsigned block = (unsigned)row_block(a0.grid_x);   // (rows, and so blocks, are below 2^31 a task)
+  if (block < blocks0) {
+    if (sums_only(a0)) inv_rms_of_sums<W>(a0, block);
+    else rms_prep_rows<NCH, W, NT>(a0, block);
   } else {
-    rms_prep_rows<NCH, W, NT>(a1, blockIdx.x - blocks0);
+    rms_prep_rows<NCH, W, NT>(a1, block - blocks0);
   }
 }
 
@@ -197,16 +201,18 @@ constexpr int64_t kStreamBytes = int64_t(128) << 20;
 
 // Launches `a0` alone (a1 null) or both tasks.
 template <int NCH, int W, bool NT>
-int launch_prep(const PrepArgs& a0, const PrepArgs* a1, hipStream_t s) {
+int launch_prep(PrepArgs a0, const PrepArgs* a1, hipStream_t s) {
   constexpr int R = rows_per_block(W);
-  const dim3 block(row_threads(W));
   const int per0 = a1 != nullptr && sums_only(a0) ? row_threads(W) : R;
-  const int blocks0 = (a0.B * a0.L + per0 - 1) / per0;
+  const int64_t blocks0 = ((int64_t)a0.B * a0.L + per0 - 1) / per0;
+  const int64_t blocks1 = a1 != nullptr ? ((int64_t)a1->B * a1->L + R - 1) / R : 0;
+  const RowGrid g = row_grid(blocks0 + blocks1, row_threads(W));
+  const dim3 grid(g.x, g.y), block(row_threads(W));
+  a0.grid_x = g.x;
   if (a1 == nullptr)
-    hipLaunchKernelGGL((rms_prep_kernel<NCH, W, NT>), dim3(blocks0), block, 0, s, a0);
+    hipLaunchKernelGGL((rms_prep_kernel<NCH, W, NT>), grid, block, 0, s, a0);
   else
-    hipLaunchKernelGGL((rms_prep2_kernel<NCH, W, NT>), dim3(blocks0 + (a1->B * a1->L + R - 1) / R), block, 0, s,
-                       a0, *a1, blocks0);
+    hipLaunchKernelGGL((rms_prep2_kernel<NCH, W, NT>), grid, block, 0, s, a0, *a1, (unsigned)blocks0);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : set_error(4, "rms_prep launch: %s", hipGetErrorString(e));
 }
@@ -226,6 +232,8 @@ int launch_prep_n(const PrepArgs& a0, const PrepArgs* a1, hipStream_t s) {
 int launch_prep_any(const PrepArgs& a0, const PrepArgs* a1, hipStream_t s) {
   const int nch = a0.H * 16;
   if (nch > 64 * kMaxChunksPerLane) return set_error(2, "rms_prep: H*128=%d channels exceeds 8192", a0.H * 128);
+  const int64_t most = std::max((int64_t)a0.B * a0.L, a1 != nullptr ? (int64_t)a1->B * a1->L : 0);
+  if (most > 0x7fffffff) return set_error(2, "rms_prep: %lld rows is too many", (long long)most);
   if (nch <= 64) return launch_prep_n<1>(a0, a1, s);
   if (nch <= 128) return launch_prep_n<2>(a0, a1, s);
   if (nch <= 256) return launch_prep_n<4>(a0, a1, s);
@@ -237,14 +245,14 @@ int launch_prep_any(const PrepArgs& a0, const PrepArgs* a1, hipStream_t s) {
 }  // namespace
 
 int launch_rms_prep(const PrepArgs& a, hipStream_t s) {
-  if (a.B * a.L == 0) return 0;
+  if ((int64_t)a.B * a.L == 0) return 0;
   return launch_prep_any(a, nullptr, s);
 }
 
 int launch_rms_prep2(const PrepArgs& a0, const PrepArgs& a1, hipStream_t s) {
   if (a0.H != a1.H) return set_error(1, "rms_prep: the paired tasks differ in heads");
-  if (a0.B * a0.L == 0) return launch_rms_prep(a1, s);
-  if (a1.B * a1.L == 0) return launch_rms_prep(a0, s);
+  if ((int64_t)a0.B * a0.L == 0) return launch_rms_prep(a1, s);
+  if ((int64_t)a1.B * a1.L == 0) return launch_rms_prep(a0, s);
   return launch_prep_any(a0, &a1, s);
 }
 
