@@ -91,7 +91,8 @@ int wan_cross_attn(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out,
  * of workgroups mostly empty, their keys are split over the idle compute units, and the
  * parts' fp32 results (O, running max, row sum) are merged by a second kernel; they go to
  * `workspace`, 256-byte aligned, of wan_flash_attn_workspace() bytes (0: this size does not
- * split).  With NULL or fewer bytes the call runs unsplit, as the entry point without _ws.
+ * split).  With fewer bytes the call splits as far as they go, with NULL or too few for two
+ * parts it runs unsplit, as the entry point without _ws.
  */
 size_t wan_flash_attn_workspace(int batch, int heads, int seqlen_q, int seqlen_k);
 int wan_flash_self_attn_ws(wan_tensor q, wan_tensor k, wan_tensor v, wan_tensor out,

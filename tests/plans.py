@@ -10,6 +10,11 @@ SHIM = """
 #include "plans.h"
 using namespace wan;
 extern "C" {
+void attention(int B, int H, int Lq, int keys, int cus, size_t scratch, int* out, size_t* bytes) {
+  const SplitPlan p = split_plan(B, H, Lq, keys, cus, scratch);
+  out[0] = p.from; out[1] = p.blocks; out[2] = p.splits;
+  *bytes = p.bytes;
+}
 void rows(long long blocks, int threads, unsigned* out) {
   const RowGrid g = row_grid(blocks, threads);
   out[0] = g.x; out[1] = g.y;
@@ -46,3 +51,10 @@ def rows(lib, blocks, threads):
     out = (ctypes.c_uint * 2)()
     lib.rows(ctypes.c_longlong(blocks), threads, out)
     return tuple(out)
+
+
+def attention(lib, B, H, Lq, keys, cus=256, scratch=1 << 40):
+    """(whole blocks, split blocks, parts of each, scratch bytes)"""
+    out, n = (ctypes.c_int * 3)(), ctypes.c_size_t()
+    lib.attention(B, H, Lq, keys, cus, ctypes.c_size_t(scratch), out, ctypes.byref(n))
+    return (*out, n.value)

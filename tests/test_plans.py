@@ -47,3 +47,20 @@ def test_row_grid(lib, waves):
         assert x * threads < 2 ** 32 and y < 2 ** 16
         assert blocks <= x * y < blocks + y
         assert y == 1 or blocks > line
+
+
+def test_attention_splits_with_the_scratch_of_all_keys(lib, W):
+    """A call over the first `keys` of the tensor's keys is given the scratch of all of them (256 CUs
+    without a device): it splits as far as that goes wherever a call without a limit would."""
+    ws = W._native.lib().wan_flash_attn_workspace
+    assert plans.attention(lib, 1, 32, 256, 4100)[2] == 6 and plans.attention(lib, 1, 32, 256, 4096)[2] == 8
+    assert plans.attention(lib, 1, 32, 256, 4096, scratch=ws(1, 32, 256, 4100))[2] == 6
+    for blocks in (1, 8, 32, 33, 48, 120, 128, 200, 256 + 32, 816):
+        for keys in range(1025, 9000, 37):
+            whole = plans.attention(lib, 1, 1, 256 * blocks, keys)
+            assert whole[3] == ws(1, 1, 256 * blocks, keys)
+            for fewer in (keys - 1, keys - 64, keys - 300):
+                free = plans.attention(lib, 1, 1, 256 * blocks, fewer)
+                p = plans.attention(lib, 1, 1, 256 * blocks, fewer, scratch=whole[3])
+                assert p[3] <= whole[3] and p[2] <= free[2]
+                assert (p[2] > 1) == (free[2] > 1 and whole[2] > 1), (blocks, keys, fewer)

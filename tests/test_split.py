@@ -150,3 +150,20 @@ def test_split_fused_under_capture(W):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(captured, call())
+
+
+@pytest.mark.gpu
+def test_split_of_fewer_keys_than_the_scratch_was_sized_for(W):
+    """65 tiles in the tensor (32 blocks: six parts), 64 of them attended to (eight parts, were there room)."""
+    N, lib = W._native, W._native.lib()
+    H, Lq, Lk, n = 32, 256, 4100, 4096
+    q, k, v = _bf((1, Lq, H, D), 1), _bf((1, Lk, H, D), 2), _bf((1, Lk, H, D), 3)
+    k[:, n:], v[:, n:] = 1e4, float("nan")
+    size = lib.wan_flash_attn_workspace(1, H, Lq, Lk)
+    part, out = torch.full((size // 4 + 64,), float("nan"), device=DEV), torch.empty_like(q)
+    N.check("split", lib.wan_flash_self_attn_ws(N.tensor4(q), N.tensor4(k), N.tensor4(v), N.tensor4(out), 1, H, Lq, Lk, D,
+                                                SCALE, n, part.data_ptr(), size, torch.cuda.current_stream().cuda_stream))
+    assert not part[:size // 4].isnan().any() and part[size // 4:].isnan().all()     # it was split, within its scratch
+    want = _softmax64(q, k, v, [n])
+    e, e0 = _rel(out, want), _rel(_unsplit(W, q, k, v, None, n), want)
+    assert e <= 1.05 * e0 + 1e-5

@@ -52,14 +52,14 @@
 //    batch index varies fastest instead, balancing long and short samples
 //    over the XCDs.
 #include "common.h"
-
+#include "plans.h"
 
 namespace wan {
 
 namespace {
 
-constexpr int BN = 64;                  // keys per tile
-constexpr int kWaves = 8;               // waves per workgroup: 256 query rows, one workgroup per CU
+constexpr int BN = kTileKeys;           // keys per tile
+constexpr int kWaves = kAttnWaves;      // waves per workgroup: 256 query rows, one workgroup per CU
 constexpr int D = kHeadDim;             // 128
 constexpr int kTileElems = BN * D;      // one K or V tile: 64 rows of 256 B
 constexpr float kLog2e = 1.4426950408889634f;
@@ -481,10 +481,6 @@ __device__ __forceinline__ BlockId block_id(const FlashArgs& a, int pid, int num
   }
   return r;
 }
-
-// A split part's result: per wave (32 query rows) 16 groups of 64 x 4 fp32 (group 4 md + g
-// holds o[md][4g..4g+3] of every lane, so that one store writes 1 KB), then m and l per lane.
-constexpr int kPartFloats = 64 * 64 + 128;
 
 template <int NW, int QP, bool SPLIT>
 __global__ __launch_bounds__(NW * 64, 2) void flash_fwd_kernel(const FlashArgs a) {
@@ -1062,41 +1058,6 @@ int launch_short(const FlashArgs& a, hipStream_t s) {
 // tiles (measured 5% faster at 512 keys; equal or slower from 1080 keys on).
 constexpr int kShortKeys = 1024;
 
-// How the 8-wave kernel's last round of workgroups (one per CU) is split.  When the blocks
-// leave `rem` of them for a last round and that fills half of the CUs at most, each of
-// those is run as n workgroups over a part of the keys and merged.  A tile less costs ~1.4 us
-// less; a split costs ~5 us (the merge launch, the parts' own start) and 0.05 us per part
-// (132 KB of fp32 written and read).  Self-attention, batch 2, 24 heads, us unsplit / split:
-//   1500 tokens (rem 32, n 8)  107.6 / 92.6      2048 (rem 128, n 2)  139.4 / 132.8
-//   4114 (rem 48, n 5)         482.1 / 437.3
-// More than one round of parts loses: 4862 tokens (rem 144) 576 / 581 at n 3, 7854 (rem 208)
-// 1382 / 1411 at n 2 -- while a last round is partly idle the busy CUs clock higher.
-struct SplitPlan {
-  int from, blocks, splits;   // whole blocks, split blocks, parts of each
-  size_t bytes;
-};
-constexpr int kMaxSplits = 8;
-SplitPlan split_plan(int B, int H, int Lq, int Lk) {
-  SplitPlan p{0, 0, 1, 0};
-  const int64_t blocks = (int64_t)((Lq + kWaves * 32 - 1) / (kWaves * 32)) * B * H;
-  const int cus = device_cu_count();
-  const int rem = (int)(blocks % cus), nt = (Lk + BN - 1) / BN;
-  if (rem == 0 || blocks > 0x7fffffff) return p;
-  float best = 0.f;
-  for (int n = 2; n <= kMaxSplits && rem * n <= cus && n <= nt; ++n) {
-    const float gain = 1.4f * (nt - (nt + n - 1) / n) - 5.f - 0.05f * (rem * n);
-    if (gain > best) {
-      best = gain;
-      p.splits = n;
-    }
-  }
-  if (p.splits < 2) return p;
-  p.from = (int)(blocks - rem);
-  p.blocks = rem;
-  p.bytes = (size_t)rem * p.splits * kWaves * kPartFloats * sizeof(float);
-  return p;
-}
-
 template <int NW, int QP>
 int launch_nw(const FlashArgs& a, hipStream_t s) {
   constexpr int BM = NW * 32;
@@ -1104,8 +1065,9 @@ int launch_nw(const FlashArgs& a, hipStream_t s) {
   const int64_t grid = num_m * a.B * a.H;
   if (grid > 0x7fffffff) return set_error(2, "flash_fwd: grid of %lld workgroups too large", (long long)grid);
   if constexpr (NW == kWaves) {
-    const SplitPlan p = split_plan(a.B, a.H, a.Lq, a.seqlen_k != nullptr ? a.Lk : a.seqlen_all);
-    if (p.splits > 1 && a.part != nullptr && a.part_bytes >= p.bytes) {
+    const SplitPlan p = split_plan(a.B, a.H, a.Lq, a.seqlen_k != nullptr ? a.Lk : a.seqlen_all, device_cu_count(),
+                                   a.part != nullptr ? a.part_bytes : 0);
+    if (p.splits > 1) {
       FlashArgs as = a;
       as.split_from = p.from;
       as.splits = p.splits;
@@ -1159,7 +1121,7 @@ int device_cu_count() {
 
 size_t flash_split_bytes(int B, int H, int Lq, int Lk) {
   if (B <= 0 || H <= 0 || Lq <= 0 || Lk <= kShortKeys) return 0;
-  return split_plan(B, H, Lq, Lk).bytes;
+  return split_plan(B, H, Lq, Lk, device_cu_count(), SIZE_MAX).bytes;
 }
 
 int launch_flash_fwd(const FlashArgs& a, hipStream_t s) {

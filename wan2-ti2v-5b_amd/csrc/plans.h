@@ -8,6 +8,52 @@
 namespace wan {
 
 // ---------------------------------------------------------------------------
+// the attention (flash_fwd.hip)
+// ---------------------------------------------------------------------------
+
+constexpr int kAttnWaves = 8, kTileKeys = 64;   // waves per workgroup (32 query rows each), keys per tile
+// A split part's result: per wave (32 query rows) 16 groups of 64 x 4 fp32 (group 4 md + g
+// holds o[md][4g..4g+3] of every lane, so that one store writes 1 KB), then m and l per lane.
+constexpr int kPartFloats = 64 * 64 + 128;
+
+// How the 8-wave kernel's last round of workgroups (one per CU) is split.  When the blocks
+// leave `rem` of them for a last round and that fills half of the CUs at most, each of
+// those is run as n workgroups over a part of the keys and merged.  A tile less costs ~1.4 us
+// less; a split costs ~5 us (the merge launch, the parts' own start) and 0.05 us per part
+// (132 KB of fp32 written and read).  Self-attention, batch 2, 24 heads, us unsplit / split:
+//   1500 tokens (rem 32, n 8)  107.6 / 92.6      2048 (rem 128, n 2)  139.4 / 132.8
+//   4114 (rem 48, n 5)         482.1 / 437.3
+// More than one round of parts loses: 4862 tokens (rem 144) 576 / 581 at n 3, 7854 (rem 208)
+// 1382 / 1411 at n 2 -- while a last round is partly idle the busy CUs clock higher.
+// The best n is not monotone in the keys (rem 32: 65 tiles in 6 parts, 64 in 8), and the scratch was
+// sized for all keys of the tensor where the launch may be given fewer: n is what `scratch` holds.
+struct SplitPlan {
+  int from, blocks, splits;   // whole blocks, split blocks, parts of each
+  size_t bytes;
+};
+constexpr int kMaxSplits = 8;
+inline SplitPlan split_plan(int B, int H, int Lq, int keys, int cus, size_t scratch) {
+  SplitPlan p{0, 0, 1, 0};
+  const int64_t blocks = (int64_t)((Lq + kAttnWaves * 32 - 1) / (kAttnWaves * 32)) * B * H;
+  const int rem = (int)(blocks % cus), nt = (keys + kTileKeys - 1) / kTileKeys;
+  if (rem == 0 || blocks > 0x7fffffff) return p;
+  const size_t part = (size_t)rem * kAttnWaves * kPartFloats * sizeof(float);   // bytes, one part of each block
+  float best = 0.f;
+  for (int n = 2; part * n <= scratch && n <= kMaxSplits && rem * n <= cus && n <= nt; ++n) {
+    const float gain = 1.4f * (nt - (nt + n - 1) / n) - 5.f - 0.05f * (rem * n);
+    if (gain > best) {
+      best = gain;
+      p.splits = n;
+    }
+  }
+  if (p.splits < 2) return p;
+  p.from = (int)(blocks - rem);
+  p.blocks = rem;
+  p.bytes = part * p.splits;
+  return p;
+}
+
+// ---------------------------------------------------------------------------
 // the token-row kernels (prep.hip, adaln.hip)
 // ---------------------------------------------------------------------------
 
