@@ -167,3 +167,24 @@ def test_split_of_fewer_keys_than_the_scratch_was_sized_for(W):
     want = _softmax64(q, k, v, [n])
     e, e0 = _rel(out, want), _rel(_unsplit(W, q, k, v, None, n), want)
     assert e <= 1.05 * e0 + 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("low", [float("-inf"), -3e38])
+@pytest.mark.parametrize("first,last", [(64, 1500), (200, 1500), (700, 1300), (0, 700)])
+def test_split_with_scores_of_minus_infinity(W, low, first, last):
+    """Keys whose scores are -inf weigh nothing, also where a part's first tile, or all of a part, has no
+    others; a first tile without others gives NaN, split or not."""
+    B, H, Lq, Lk = 2, 3, 257, 1500
+    assert W._native.lib().wan_flash_attn_workspace(B, H, Lq, Lk) > 0
+    q, k, v = _bf((B, Lq, H, D), 1).abs() + 1, _bf((B, Lk, H, D), 2), _bf((B, Lk, H, D), 3)
+    k[:, first:last] = low
+    out, whole = W.ops.flash_self_attn(q, k, v, SCALE, 0), _unsplit(W, q, k, v, None)
+    if first == 0:
+        assert out.isnan().all() and whole.isnan().all()
+        return
+    keep = torch.cat([torch.arange(first), torch.arange(last, Lk)]).to(DEV)
+    want = _softmax64(q, k[:, keep], v[:, keep], [len(keep)] * B)
+    e, e0 = _rel(out, want), _rel(whole, want)
+    print(f"{low} at {first}..{last}: split {e:.3e}, unsplit {e0:.3e}")
+    assert e <= 1.05 * e0 + 1e-5

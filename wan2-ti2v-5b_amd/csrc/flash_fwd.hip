@@ -54,6 +54,8 @@
 #include "common.h"
 #include "plans.h"
 
+#include <cfloat>
+
 namespace wan {
 
 namespace {
@@ -665,6 +667,9 @@ __global__ __launch_bounds__(NW * 64, 2) void flash_fwd_kernel(const FlashArgs a
       __syncthreads();  // every wave is done with K0 before it is overwritten
     }
 
+    // A part that begins with a tile of scores -inf (which weigh nothing in a launch that is not
+    // split, there being finite ones before them) needs a finite reference point for them.
+    if (SPLIT && key0 > 0) c.m_run = fmaxf(c.m_run, -FLT_MAX);
     int t = 0;
     const bf16* v_last = v_lds[0];
     if constexpr (RING == 2) {
