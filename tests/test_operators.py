@@ -2,9 +2,15 @@
 the operators: the same bits for ordinary calls, and everything else as the functions have it
 (errors, empty tensors, autograd, tracing, vmap).  A call whose first tensor requires a gradient
 runs the Python function."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 from torch.utils._python_dispatch import TorchDispatchMode
+
+import __graft_entry__
 
 B, L, H, D = 2, 37, 24, 128
 C = H * D
@@ -158,3 +164,54 @@ def test_linear_misaligned_is_torchs(W, which):
         if off % 8:
             assert torch.equal(W.ops.linear(**args), torch.nn.functional.linear(**{"input": args["x"], "weight": args["weight"],
                                                                                      "bias": args["bias"]}))
+
+
+def _fresh(code, tmp_path):
+    """Runs code in a new process over a copy of the package's Python files in tmp_path."""
+    import shutil
+    for f in os.listdir(__graft_entry__.PKG_DIR):
+        if f.endswith(".py") or f == "libwan_attn.so":
+            shutil.copy(os.path.join(__graft_entry__.PKG_DIR, f), tmp_path)
+    code = (f"import sys, warnings, torch; sys.path.insert(0, {__graft_entry__.ROOT!r})\n"
+            f"import __graft_entry__ as g; g.PKG_DIR = {str(tmp_path)!r}\n" + code)
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr
+    return r.stdout
+
+
+def test_import_with_operators_that_do_not_load(tmp_path):
+    """The package imports and its torch side runs; the first kernel call says what is wrong."""
+    (tmp_path / f"libwan_ops-torch{torch.__version__}.so").write_bytes(b"not a library")
+    (tmp_path / "libwan_ops.so").write_bytes(b"not a library")
+    out = _fresh("""W = g.load_package()
+m = W.model.random_model(W.model.WanConfig(dim=256, ffn_dim=512, num_heads=2, num_layers=1, in_dim=4, out_dim=4,
+                                           text_dim=64, freq_dim=32), device="cpu", std=0.05)
+fast = W.fast_dit.FastWanDiT(m, (1, 2, 2), 5.0, "sdpa", "sdpa", "eager")
+fast.set_context(torch.zeros(1, 3, 64), torch.zeros(1, 3, 64))
+print(tuple(fast(torch.zeros(4, 1, 4, 4), 1).shape))
+try:
+    W._native.lib()
+except RuntimeError as e:
+    print("does not load" in str(e))
+""", tmp_path)
+    assert out.split("\n")[:2] == ["(4, 1, 4, 4)", "True"]
+
+
+def test_import_with_another_torch(tmp_path):
+    """With operators built for another torch, which are not loaded, the Python functions are there, with
+    a warning; with none built at all the first kernel call raises."""
+    (tmp_path / "libwan_ops-torch0.1.so").write_bytes(b"not for this torch")
+    out = _fresh("""W = g.load_package()
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    print(W._native.lib().wan_attn_abi_version(), len([w for w in seen if "another torch" in str(w.message)]))
+""", tmp_path)
+    assert out.split() == ["1", "1"]
+    (tmp_path / "libwan_ops-torch0.1.so").unlink()
+    out = _fresh("""W = g.load_package()
+try:
+    W._native.lib()
+except RuntimeError as e:
+    print("not built" in str(e))
+""", tmp_path)
+    assert out.split() == ["True"]

@@ -1,5 +1,5 @@
 """ctypes binding of libwan_attn.so, the C ABI declared in include/wan_attn.h, and the loading of
-libwan_ops.so, the torch operators' native kernels over it.
+libwan_ops, the torch operators' native kernels over it, built for one torch.
 
 torch is imported first on purpose: the library is linked against the HIP
 runtime by soname (libamdhip64.so.7), and the dynamic loader resolves that to
@@ -9,12 +9,14 @@ no fallback path.
 """
 import ctypes
 import os
+import warnings
 
 import torch  # (must precede the CDLL load, see above)
 
 LIB_NAME = "libwan_attn.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
-OPS_LIB_PATH = os.path.join(os.path.dirname(LIB_PATH), "libwan_ops.so")
+OPS_LIB_NAME = f"libwan_ops-torch{torch.__version__}.so"      # built for this torch (build.py)
+OPS_LIB_PATH = os.path.join(os.path.dirname(LIB_PATH), OPS_LIB_NAME)
 
 
 class WanTensor(ctypes.Structure):
@@ -65,17 +67,25 @@ SIGNATURES = {
 ABI_VERSION = 1
 
 _lib = None
+_ops_error = None
 
 
 def lib() -> ctypes.CDLL:
     """The loaded library (loaded on first use). Raises if it is missing or stale."""
     global _lib
     if _lib is None:
-        missing = [p for p in (LIB_PATH, OPS_LIB_PATH) if not os.path.exists(p)]
+        # built for another torch, the operators run as without their native kernels
+        built = [f for f in os.listdir(os.path.dirname(OPS_LIB_PATH)) if f.startswith("libwan_ops-torch")]
+        missing = [p for p, there in ((LIB_PATH, os.path.exists(LIB_PATH)), (OPS_LIB_PATH, built)) if not there]
         if missing:
             raise RuntimeError(
                 f"{' and '.join(missing)} not built; run `python __graft_entry__.py build` "
                 "(or wan2-ti2v-5b_amd/build.py) first")
+        if _ops_error is not None:
+            raise RuntimeError(f"{OPS_LIB_PATH} does not load: {_ops_error}")
+        if not os.path.exists(OPS_LIB_PATH):
+            warnings.warn(f"the torch operators' native kernels are built for another torch than {torch.__version__} "
+                          f"({', '.join(built)}): calls take the Python functions, with more host time; build again")
         handle = ctypes.CDLL(LIB_PATH)
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(handle, name)
@@ -88,10 +98,15 @@ def lib() -> ctypes.CDLL:
 
 
 def load_operators() -> None:
-    """Registers the operators' native kernels, once ops.py has defined the operators.  Before the
-    libraries are built there is nothing to register: the first call raises in lib()."""
+    """Registers the operators' native kernels, once ops.py has defined the operators.  Importing the
+    package asks for neither library, nor for the torch that one was built for: what is missing or does
+    not load is told by the first kernel call, in lib()."""
+    global _ops_error
     if os.path.exists(LIB_PATH) and os.path.exists(OPS_LIB_PATH):
-        torch.ops.load_library(OPS_LIB_PATH)
+        try:
+            torch.ops.load_library(OPS_LIB_PATH)
+        except OSError as e:
+            _ops_error = str(e)
 
 
 def last_error() -> str:

@@ -1,5 +1,5 @@
 """Build recipe for libwan_attn.so, the gfx950 HIP kernels behind include/wan_attn.h, and for
-libwan_ops.so, the torch operators' native kernels that call it (host code).
+libwan_ops-torch<version>.so, the torch operators' native kernels that call it (host code).
 
 Each csrc/*.hip file is compiled with hipcc for gfx950 only, in parallel, and
 the objects are linked into one shared library next to this file (in-tree, so
@@ -21,8 +21,6 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 BUILD_DIR = os.path.join(PKG_DIR, "_build")
 LIB_NAME = "libwan_attn.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
-OPS_LIB_NAME = "libwan_ops.so"
-OPS_LIB_PATH = os.path.join(PKG_DIR, OPS_LIB_NAME)
 ARCH = "gfx950"
 
 HIPCC = os.environ.get("HIPCC", os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "bin", "hipcc"))
@@ -53,6 +51,12 @@ def _run(cmd):
     return out
 
 
+def _ops_lib_path():
+    """The torch operators' library: named for the torch that it is built against, which alone loads it."""
+    import torch
+    return os.path.join(PKG_DIR, f"libwan_ops-torch{torch.__version__}.so")
+
+
 def _ops_commands(obj, out):
     """Compile and link commands of the torch operators."""
     import torch
@@ -69,7 +73,7 @@ def _ops_commands(obj, out):
 
 
 def build(verbose: bool = False) -> str:
-    """Compile every HIP source and link libwan_attn.so, then libwan_ops.so; returns the path of the first."""
+    """Compile every HIP source and link libwan_attn.so, then the operators' library; returns the path of the first."""
     if not os.path.exists(HIPCC):
         raise RuntimeError(f"hipcc not found at {HIPCC}")
     os.makedirs(BUILD_DIR, exist_ok=True)
@@ -78,7 +82,8 @@ def build(verbose: bool = False) -> str:
     jobs = min(len(srcs) + 1, int(os.environ.get("MAX_JOBS", "8")))
     with cf.ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
         futs = [ex.submit(_run, [HIPCC, *DEVICE_FLAGS, "-c", s, "-o", o]) for s, o in zip(srcs, objs)]
-        ops_tmp = OPS_LIB_PATH + ".tmp"
+        ops_path = _ops_lib_path()
+        ops_tmp = ops_path + ".tmp"
         compile_ops, link_ops = _ops_commands(os.path.join(BUILD_DIR, "torch_ops.o"), ops_tmp)
         futs.append(ex.submit(_run, compile_ops))
         for f in futs:
@@ -89,9 +94,12 @@ def build(verbose: bool = False) -> str:
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp])
     os.replace(tmp, LIB_PATH)
     _run(link_ops)
-    os.replace(ops_tmp, OPS_LIB_PATH)
+    for f in os.listdir(PKG_DIR):
+        if f.startswith("libwan_ops") and f.endswith(".so"):      # of older sources, or for another torch
+            os.remove(os.path.join(PKG_DIR, f))
+    os.replace(ops_tmp, ops_path)
     if verbose:
-        print(f"built {LIB_PATH} and {OPS_LIB_NAME}")
+        print(f"built {LIB_PATH} and {os.path.basename(ops_path)}")
     return LIB_PATH
 
 
