@@ -10,7 +10,8 @@
     computes them from the rows (the fp32 sum order differs: equal up to rare one-ulp flips
     before the rotation, bounded against each rotated pair's norm), and against the oracle
     (oracle.inv_rms, oracle.rms, oracle.rope) on the GEMM's own q and k;
-  * a whole WanAttentionBlock with FAST_QKV_IMPL "hip" against the default "hipblaslt".
+  * a whole WanAttentionBlock with FAST_QKV_IMPL "hip" against "hipblaslt", and the default "auto" against
+    both on either side of where it changes between them.
 """
 import pytest
 import torch
@@ -146,3 +147,24 @@ def test_block_with_qkv_sumsq_matches_default(W):
     e = ref.rel_rms(outs["hip"].cpu(), outs["hipblaslt"].cpu())
     print(f"block with the sums-of-squares GEMM vs hipBLASLt projection: rel_rms {e:.3e}")
     assert torch.isfinite(outs["hip"]).all() and e < 1e-3
+
+
+@pytest.mark.parametrize("grid,own", [((6, 12, 15), True), ((1, 28, 40), True), ((1, 19, 59), False)])
+def test_block_auto_is_one_of_the_two(W, grid, own):
+    """2160, 2240 and 2242 tokens of both samples: the bits of the "hip" route up to 2240, from there on
+    "hipblaslt"'s.  The two are results of the same values, one bf16 rounding (2^-8 relative at most) apart
+    where they differ at all."""
+    m = W.model.random_model(W.model.WanConfig(), num_layers=1, device=DEV, seed=11)
+    L = grid[0] * grid[1] * grid[2]
+    g = torch.Generator().manual_seed(L)
+    x = torch.randn(2, L, 3072, generator=g).bfloat16().to(DEV)
+    e0 = (torch.randn(1, grid[0], 6, 3072, generator=g) * 0.1).bfloat16().to(DEV)
+    ctx = torch.randn(2, 77, 3072, generator=g).bfloat16().to(DEV)
+    cos, sin = W.rope.rope_tables(m.freqs, grid, 128, DEV)
+    ck, cv = W.fast_dit.cross_kv(m.blocks[0], ctx, "hip")
+    outs = {impl: W.fast_dit._FastBlock(m.blocks[0], grid[0], "hip", "hip", "hip", impl)(x, e0, cos, sin, ck, cv)
+            for impl in ("auto", "hip", "hipblaslt")}
+    assert torch.isfinite(outs["auto"]).all()
+    assert torch.equal(outs["auto"], outs["hip" if own else "hipblaslt"])
+    e = ref.rel_rms(outs["hip"].float().cpu(), outs["hipblaslt"].float().cpu())
+    assert e <= 2 ** -8, e

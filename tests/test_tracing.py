@@ -1,5 +1,6 @@
 """Tracing of a whole WanAttentionBlock (torch.compile with fullgraph, plain fake tensors), on fake
 device tensors: no kernel runs and no device is needed."""
+import collections
 import warnings
 
 import pytest
@@ -65,10 +66,10 @@ def test_block_on_fake_tensors(W, tokens, frames):
 class _Names(TorchDispatchMode):
     def __init__(self):
         super().__init__()
-        self.names = set()
+        self.count = collections.Counter()
 
     def __torch_dispatch__(self, func, types, args=(), kwargs=None):
-        self.names.add(str(func))
+        self.count[str(func)] += 1
         return func(*args, **(kwargs or {}))
 
 
@@ -90,10 +91,32 @@ def test_torch_side_runs_torch_alone(W, impl, pointwise, monkeypatch):
             _, args = _block(W, 2160, grid[0])
             with _Names() as seen:
                 fast.time_rows(500)
-                before = {n for n in seen.names if n.startswith("wan_hip.")}
+                before = {n for n in seen.count if n.startswith("wan_hip.")}
                 fb(*args)
     finally:
         torch.set_default_dtype(torch.float32)
     assert not before
-    own = {n for n in seen.names if n.startswith("wan_hip.")}
+    own = {n for n in seen.count if n.startswith("wan_hip.")}
     assert bool(own) == (impl == "hip"), own
+
+
+# the ends of the ranges in which a projection is this library's: (tokens of both samples, q/k/v, the
+# 3072-wide ones, FFN-down); odd counts do not occur with guidance
+@pytest.mark.parametrize("tokens,qkv,wide,down", [
+    (2, 0, 0, 0), (64, 0, 0, 0), (66, 0, 0, 1), (1080, 0, 0, 1), (1792, 0, 0, 1), (1794, 0, 0, 0), (1822, 0, 0, 0),
+    (1824, 1, 0, 0), (2110, 1, 0, 0), (2160, 1, 0, 1), (2240, 1, 0, 1), (2242, 0, 0, 1), (2306, 0, 0, 0),
+    (5470, 0, 0, 0), (5504, 1, 1, 1), (5888, 1, 1, 1), (6656, 0, 1, 0), (6658, 0, 0, 0), (8704, 1, 0, 1),
+    (12288, 1, 0, 0), (14336, 0, 0, 1), (14338, 0, 0, 0), (15708, 0, 0, 0)])
+def test_projection_routes(W, tokens, qkv, wide, down):
+    with FakeTensorMode(), torch.no_grad():
+        fb, args = _block(W, tokens, 1)
+        with _Names() as seen:
+            fb(*args)
+        assert seen.count["wan_hip.qkv_proj_sumsq.default"] == qkv
+        assert seen.count["wan_hip.self_attn_fused_sumsq.default"] == qkv
+        assert seen.count["wan_hip.linear.default"] == 3 * wide + down
+        for impl, calls in (("hipblaslt", 0), ("hip", 1)):      # chosen by name: at every size
+            fb.qkv_impl = impl
+            with _Names() as seen:
+                fb._self_attention(args[0], args[2], args[3])
+            assert seen.count["wan_hip.qkv_proj_sumsq.default"] == calls

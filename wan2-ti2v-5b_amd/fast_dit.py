@@ -48,7 +48,7 @@ FAST_POINTWISE_IMPL = os.environ.get("FAST_POINTWISE_IMPL", "hip")
 # The fused q/k/v projection of the "hip" self-attention: "hipblaslt", or "hip", the gfx950 GEMM
 # whose epilogue emits the QK-RMSNorm sums of squares (ops.qkv_proj_sumsq), so the q statistics
 # pass disappears, or "auto" (default), "hip" at the token counts where that GEMM is the faster
-# one (_OWN_GEMM_ROWS; at the B=2, L=7854 shape it takes 0.69 ms against hipBLASLt's 0.61).
+# one (_OWN_GEMM_ROWS; at the B=2, L=7854 shape it takes 0.68 ms against hipBLASLt's 0.62).
 FAST_QKV_IMPL = os.environ.get("FAST_QKV_IMPL", "auto")
 IMPLS = ("hip", "sdpa")
 for _name, _val in (("FAST_ATTN_IMPL", FAST_ATTN_IMPL), ("FAST_CROSS_IMPL", FAST_CROSS_IMPL)):
@@ -137,22 +137,31 @@ def _ffn_gelu_epilogue(h, ffn):
 
 
 # Rows (tokens of all samples) at which the projection from k to n channels is taken to this
-# library's GEMM (ops.linear).  hipBLASLt's choice of kernel changes from size
-# to size, and where it takes one that neither splits nor streams k it runs the long FFN-down
+# library's GEMM (ops.linear; q, k and v ops.qkv_proj_sumsq).  hipBLASLt's choice of kernel changes
+# from size to size, and where it takes one that neither splits nor streams k it runs the long FFN-down
 # product on as many CUs as it has tiles, or leaves most of the last round idle; this GEMM splits
-# those tiles.  Measured every 64 to 128 rows from 64 to 16384 with the weights from memory; inside
-# these ranges it is 4% to 45% faster, outside hipBLASLt is faster or within 5%.  us there / here:
-#   14336 -> 3072   368 77 / 48    1080 125 / 108   2160 266 / 173   4488 476 / 370   5984 753 / 417
-#                   7480 848 / 521   8976 853 / 630   9724 947 / 690   12716 1018 / 900
-#                   outside: 2600 193 / 197   3740 252 / 310   8228 591 / 576   15708 930 / 1150
-#   3072 -> 3072    2160 47 / 45   2440 51 / 46   5624 111 / 95   6246 113 / 97   outside: 2600 51 / 49
-#                   15708 207 / 248
-#   3072 -> 9216    1900 118 / 97   2160 110 / 102   5624 312 / 270   8228 445 / 375   11069 516 / 477
-#                   outside: 1720 80 / 90   4192 202 / 202   6820 290 / 324   15708 613 / 690
+# those tiles.  Measured against the hipBLASLt of torch 2.10.0+rocm7.0 at a random row count in
+# every 12 (FFN-down) or 16 from 1 to 16384, the weights from memory: inside the ranges it is
+# faster at every one of them, by 3% to 49%.  us there / here:
+#   14336 -> 3072   72 36 / 34   1080 125 / 108   2113 266 / 171   2726 370 / 219   3454 409 / 261
+#                   4598 480 / 331   5511 662 / 396   6260 452 / 411   7672 766 / 512   8590 831 / 581
+#                   10226 883 / 683   11633 1095 / 850   14331 1147 / 961
+#   3072 -> 3072    5516 107 / 84   6645 102 / 94
+#   3072 -> 9216    1827 105 / 84   2228 105 / 95   5483 297 / 258   5879 311 / 261   7564 385 / 349
+#                   8702 463 / 373   10885 507 / 462   12285 598 / 540
+# Most of the ends are where hipBLASLt changes its kernel, and it is the faster past them: 14336 -> 3072
+# at 1 to 63 rows (21 rows 1.4 times), 1843 161 / 164, 2307 180 / 187, 3459 250 / 271, 4618 279 / 341,
+# 7689 508 / 537, 10245 603 / 769; 3072 -> 9216 at 2244 111 / 119, 5891 254 / 261, 8712 344 / 367, 12302
+# 487 / 541.  Others are where an earlier, coarser sweep ended, and hipBLASLt is left sizes at which
+# this GEMM would be the faster by over 5%: FFN-down 2057-2106, 2500-2558, 2700-2717, 4112-4223,
+# 5380-5501, 6274-6472, 6698-6780 (785 / 465), 8460-8569, 10949-10999, 12296-12407, 14595-15616;
+# 3072-wide 2993-3055, 5388-5499, 6660-6711, 12298-13438; q/k/v 400-448, 1805-1823, 4101-4453, 5389-5466,
+# 7438-7539, 8964-9471, 10754-10868, 13321-13554, 13838-14075.  At 15708 rows hipBLASLt is the faster for all
+# three: 920 / 1180, 208 / 229, 619 / 681.
 _OWN_GEMM_ROWS = {
-    (14336, 3072): ((1, 1856), (2112, 2304), (2720, 2848), (3376, 3456), (4224, 4608), (5504, 6272), (6784, 7680),
+    (14336, 3072): ((65, 1792), (2112, 2304), (2720, 2848), (3376, 3456), (4224, 4608), (5504, 6272), (6784, 7680),
                     (8576, 10240), (11008, 11648), (12416, 14336)),
-    (3072, 3072): ((2112, 2480), (5504, 6656)),
+    (3072, 3072): ((5504, 6656),),
     (3072, 9216): ((1824, 2240), (5472, 5888), (7552, 8704), (10880, 12288)),   # q, k and v
 }
 
