@@ -258,10 +258,16 @@ def bench_cross(torch, W, dev, steps, warmup):
     }, host
 
 
+def gemm_scratch(torch, lib, M, N, K, dev):
+    """The scratch that ops.qkv_proj_sumsq gives the projection GEMM, which takes its split plan with it."""
+    n = lib.wan_qkv_proj_workspace(M, N, K)
+    return torch.empty(max(n, 1), dtype=torch.uint8, device=dev), n
+
+
 def bench_qkv(torch, W, dev, steps, warmup):
     """The block's q/k/v projection and QK-RMSNorm prep at config C (x [2, 7854, 3072],
     concatenated weight [9216, 3072]) by the two routes: hipBLASLt's GEMM, then
-    wan_rms_norm_qk (q statistics + k norm/rope from the rows); or wan_qkv_proj_sumsq, the
+    wan_rms_norm_qk (q statistics + k norm/rope from the rows); or wan_qkv_proj_sumsq_ws, the
     gfx950 GEMM that emits the sums of squares, then wan_rms_norm_qk_sumsq (no q read)."""
     import torch.nn.functional as F
     N_, lib = W._native, W._native.lib()
@@ -289,9 +295,12 @@ def bench_qkv(torch, W, dev, steps, warmup):
                                                 gk.data_ptr(), 1e-6, cos.data_ptr(), sin.data_ptr(),
                                                 inv.data_ptr(), s))
 
+    ws, ws_bytes = gemm_scratch(torch, lib, B * L, 3 * C, C, dev)
+
     def gemm_sumsq():
-        N_.check("qkv gemm", lib.wan_qkv_proj_sumsq(x.data_ptr(), w.data_ptr(), bias.data_ptr(), qkv.data_ptr(),
-                                                    ss.data_ptr(), B * L, 3 * C, C, C, C, 3 * C, 2 * C, s))
+        N_.check("qkv gemm", lib.wan_qkv_proj_sumsq_ws(x.data_ptr(), w.data_ptr(), bias.data_ptr(), qkv.data_ptr(),
+                                                       ss.data_ptr(), B * L, 3 * C, C, C, C, 3 * C, 2 * C,
+                                                       ws.data_ptr(), ws_bytes, s))
 
     def prep_sums():
         N_.check("qk prep from sums", lib.wan_rms_norm_qk_sumsq(N_.tensor4(k), khat.data_ptr(), B, L, H, D,
@@ -324,9 +333,12 @@ def qkv_gemms_alone(torch, W, dev, launches):
     ss = torch.empty(4 * H, B * L, device=dev, dtype=torch.float32)
     s = torch.cuda.current_stream().cuda_stream
 
+    ws, ws_bytes = gemm_scratch(torch, lib, B * L, 3 * C, C, dev)
+
     def gemm():
-        N_.check("qkv gemm", lib.wan_qkv_proj_sumsq(x.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(),
-                                                    ss.data_ptr(), B * L, 3 * C, C, C, C, 3 * C, 2 * C, s))
+        N_.check("qkv gemm", lib.wan_qkv_proj_sumsq_ws(x.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(),
+                                                       ss.data_ptr(), B * L, 3 * C, C, C, C, 3 * C, 2 * C,
+                                                       ws.data_ptr(), ws_bytes, s))
     res = {}
     for name, fn in (("sumsq_gemm_ms", gemm), ("hipblaslt_gemm_ms", lambda: F.linear(x, w, bias))):
         res[name] = time_alone(torch, fn, launches)

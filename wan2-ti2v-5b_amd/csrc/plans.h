@@ -112,8 +112,8 @@ struct GemmPlan {
 // round leaves half of the CUs or more idle, its tiles may be split over k: the parts' fp32 sums
 // cost a merge launch and their way through memory.  us, tiles of 256 rows alone / as chosen here:
 //   N 9216, K 3072:   M 80  56 / 23   M 256  58 / 28   M 896  60 / 46   M 2170  136 / 98 (320 rows)
-//                     M 2280  136 / 124 (a tail of 68 tiles, three parts)   M 2940  145 (256 rows)
-//                     M 4480  222 / 194 (320)   M 8228  370 / 358 (320)   M 15708  702 / 684
+//                     M 2280  136 / 120 (a tail of 68 tiles, three parts)   M 2940  143 (256 rows)
+//                     M 4480  222 / 185 (320)   M 8228  375 / 360 (320)   M 15708  690 / 680
 //   N 3072, K 14336 (the best height unsplit / as chosen):   M 80  182 / 36   M 748  178 / 82
 //                     M 1500  173 / 132   M 2160  187 / 172 (320 rows, three parts)   M 8228  739 / 581
 inline GemmPlan gemm_plan(int M, int N, int K, int64_t ldx, int cus, size_t scratch) {
