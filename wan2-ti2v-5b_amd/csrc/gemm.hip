@@ -29,9 +29,8 @@
 //
 // At the QKV shape (M 15708, N 9216, K 3072) it takes 0.67-0.69 ms as the operators run it (320 rows,
 // the tail split over k), 1.29-1.33 PFLOP/s and 88-90% of hipBLASLt's F.linear timed beside it; without
-// scratch (256 rows) 0.68-0.70 ms, and 0.745 where the pass before it has read 190 MB through the
-// caches (0.69 with the scratch: taller tiles read x and w less often).  At M 2160 (320 rows) 1.29
-// PFLOP/s against hipBLASLt's 1.17.  Both are power
+// scratch (256 rows) 0.68-0.70 ms.  At M 2160 (320 rows) 1.29 PFLOP/s against hipBLASLt's 1.17.  Both
+// are power
 // limited (all-zero operands run either ~25% faster); on zeros this kernel's k-loop is
 // ~13% slower per tile than hipBLASLt's.  4 waves of 128 x 128 (a third less LDS read
 // traffic, one wave per SIMD) run the loop at a higher clock (1.72 vs 1.58 GHz) but in

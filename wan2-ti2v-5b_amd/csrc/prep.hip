@@ -48,7 +48,15 @@ __device__ __forceinline__ void rope8(float u[8], const f32x4 c, const f32x4 s) 
 // and the launch does not end with their write-back (norm + rotation 2160 rows 8.4 -> 7.0 us,
 // 8228 rows 22.0 -> 20.1); with more than the last-level cache takes of rows read and written
 // they cost (15708 rows 36.6 -> 38.9).
-template <int NCH, int W, bool NT>
+// NTR: non-temporal reads of the rows, in the launches of both tasks that write too much to keep (q,
+// k and the written k are 289 MB at 15708 rows, the last-level cache is 256 MB).  Plain reads take
+// lines there that others have written, which must go to memory first, and put out what the next
+// kernel would have found.  15708 rows, us plain / so: the pass behind 512 MB of other writes 93 / 54, behind
+// a GEMM of other rows 61 / 53, the projection GEMM (256 rows, unsplit) behind the pass 749 / 684; behind the
+// rows' own projection, with the attention after it, 1337 / 1338.  Smaller launches, and the statistics
+// alone, read plainly: the attention finds q in the cache (2 x 1080 tokens, pass and attention
+// 53.1 / 54.0 us; statistics and cross-attention of 15708 rows 135.9 / 138.1).
+template <int NCH, int W, bool NT, bool NTR>
 __device__ __forceinline__ void rms_prep_rows(const PrepArgs& a, unsigned block) {
   const int t = W == 1 ? threadIdx.x & 63 : threadIdx.x;
   const unsigned row_id = W == 1 ? block * 4 + (threadIdx.x >> 6) : block;
@@ -66,7 +74,10 @@ __device__ __forceinline__ void rms_prep_rows(const PrepArgs& a, unsigned block)
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       const int c = t + 64 * W * i;
-      if (c < nchunks) xv[i] = *reinterpret_cast<const bf16x8*>(row + (c >> 4) * a.x.sh + (c & 15) * 8);
+      if (c < nchunks) {
+        const bf16x8* xp = reinterpret_cast<const bf16x8*>(row + (c >> 4) * a.x.sh + (c & 15) * 8);
+        xv[i] = NTR ? __builtin_nontemporal_load(xp) : *xp;
+      }
     }
   }
   // the channel pairs of a lane's chunks are the same in every head: 64 W is a multiple of 16
@@ -153,7 +164,7 @@ __device__ __forceinline__ void inv_rms_of_sums(const PrepArgs& a, unsigned bloc
 
 template <int NCH, int W, bool NT>
 __global__ __launch_bounds__(row_threads(W)) void rms_prep_kernel(const PrepArgs a) {
-  rms_prep_rows<NCH, W, NT>(a, (unsigned)row_block(a.grid_x));
+  rms_prep_rows<NCH, W, NT, false>(a, (unsigned)row_block(a.grid_x));
 }
 
 // Two independent tasks (the q statistics and the k norm + rotation of one
@@ -164,9 +175,9 @@ __global__ __launch_bounds__(row_threads(W)) void rms_prep2_kernel(const PrepArg
   const unsigned block = (unsigned)row_block(a0.grid_x);   // (rows, and so blocks, are below 2^31 a task)
   if (block < blocks0) {
     if (sums_only(a0)) inv_rms_of_sums<W>(a0, block);
-    else rms_prep_rows<NCH, W, NT>(a0, block);
+    else rms_prep_rows<NCH, W, NT, !NT>(a0, block);
   } else {
-    rms_prep_rows<NCH, W, NT>(a1, block - blocks0);
+    rms_prep_rows<NCH, W, NT, !NT>(a1, block - blocks0);
   }
 }
 
@@ -196,7 +207,8 @@ __global__ __launch_bounds__(256) void rope_kernel(const RopeArgs a) {
 
 // Up to this many rows in a launch a lane has one chunk of 8 channels, beyond it two.
 constexpr int kFewRows = 1024;
-// Normalised rows leave with plain stores when rows read and written exceed this many bytes.
+// Normalised rows leave with plain stores when rows read and written exceed this many bytes, and the
+// launches of both tasks then read non-temporally.
 constexpr int64_t kStreamBytes = int64_t(128) << 20;
 
 // Launches `a0` alone (a1 null) or both tasks.
