@@ -112,6 +112,17 @@ def test_native_equals_python(W, name):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("name", NAMES)
+def test_none_for_a_tensor_is_told_by_the_function(W, name):
+    """In place of every required tensor, the other arguments being ordinary ones: the Python function's
+    error, never one about an undefined tensor."""
+    op, args = _calls(W, "cuda", lambda shape, dtype: torch.zeros(shape, dtype=dtype, device="cuda"))[name]
+    for i in [i for i, a in enumerate(op._opoverload._schema.arguments) if str(a.type) == "Tensor"]:
+        with pytest.raises((TypeError, ValueError, AttributeError), match="None|must be a"):
+            op(*args[:i], None, *args[i + 1:])
+
+
+@pytest.mark.gpu
 def test_other_calls_as_the_functions_have_them(W):
     o, dev = W.ops, "cuda"
     x = torch.randn(2, 5, 2, D, device=dev).bfloat16()

@@ -72,6 +72,17 @@ struct Call {
   }
 };
 
+// A kernel behind the check that every tensor is one: None for a tensor that is not optional arrives
+// as an undefined one, and the Python function says so.
+template <void (*kernel)(const OperatorHandle&, DispatchKeySet, Stack*)>
+void defined(const OperatorHandle& op, DispatchKeySet ks, Stack* stack) {
+  for (size_t i = stack->size() - op.schema().arguments().size(); i < stack->size(); ++i) {
+    const IValue& v = (*stack)[i];
+    if (v.isTensor() && !v.toTensor().defined()) return to_python(op, ks, stack);
+  }
+  kernel(op, ks, stack);
+}
+
 bool plain(const Tensor& t, at::ScalarType type, c10::Device dev) {
   return t.layout() == at::kStrided && t.scalar_type() == type && t.device() == dev;
 }
@@ -388,7 +399,7 @@ void linear(const OperatorHandle& op, DispatchKeySet ks, Stack* stack) {
   X("adaln", adaln) X("qkv_proj_sumsq", qkv_proj_sumsq) X("linear", linear)
 
 TORCH_LIBRARY_IMPL(wan_hip, CUDA, m) {
-#define WAN_IMPL(name, fn) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&fn>());
+#define WAN_IMPL(name, fn) m.impl(name, torch::CppFunction::makeFromBoxedFunction<&defined<&fn>>());
   WAN_OPS(WAN_IMPL)
 #undef WAN_IMPL
 }
